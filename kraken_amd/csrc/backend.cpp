@@ -306,6 +306,69 @@ int krk_gemm_k_ok(const krk_backend *b, int64_t k) {
 
 namespace {
 
+// Calls the weight-streaming rows kernel takes (gemm_rows.hip): 2..8 rows
+// under every path (exact products: f32 activations as two f16 planes), 9..32
+// where the path forms f16 products.  Measured against the kernels that had
+// them (us, f16 activations, 4096 -> 14336 and 14336 -> 4096):
+//   2..8 rows: Q4_K 6 rows 15.9 (17.6) and 20.7 (61.0), 4 rows 15.7 (12.5) and
+//     20.5 (41.1): the streaming GEMV keeps up to five rows of K <= 8192 and
+//     up to three of wider rows; Q6_K 2 rows 25.1 (19.5), 3 rows 24.8 (34.2)
+//     and 29.7 (45.4); Q5_K, Q8_0 and Q4_0 likewise from 3 rows;
+//   9..16: Q4_K 12 rows 16.3 (18.0) and 21.0 (20.7), Q5_K 20.7 (29.7) and 24.1
+//     (32.2), Q4_0 20.8 (32.4) and 25.0 (35.1), Q6_K 25.0 (27.6) and 30.2
+//     (30.9), Q8_0 31.8 (29.9) and 35.6 (32.8);
+//   17..32 (two passes): the dense GEMM's 64-row items win on large matrices
+//     (Q4_K 22.1 against 20.5), the rows kernel on those that leave its grid
+//     short of workgroups (2048 x 2048 8.5 against 11.5), and for Q5_K and
+//     Q4_0, whose decode to f16 values is the dearer one (28.2 against 32.2).
+constexpr int64_t kRowsExact = 8, kRowsMax = 32;
+bool rows_path(const krk_backend *b, int wt, int64_t n_out, int64_t n_in, int64_t rows, const void *w) {
+    if (rows < 2 || rows > kRowsMax) return false;
+    if (rows <= kRowsExact) {
+        if (rows < (wt == KRK_DT_Q4_K ? (n_in <= 8192 ? 6 : 4) : 3)) return false;
+    } else {
+        if (b->path != KRK_PATH_AUTO && b->path != KRK_PATH_MFMA) return false;
+        if (wt == KRK_DT_Q8_0 && n_out * n_in > (int64_t{1} << 25)) return false;
+        if (rows > 16 && n_out * n_in > (int64_t{1} << 23) &&
+            (n_in > 4096 || (wt != KRK_DT_Q5_K && wt != KRK_DT_Q4_0)))
+            return false;
+    }
+    return krk::gemm_rows_ok(wt, n_in, w, krk_dtype_row_bytes(wt, n_in)) &&
+           krk::gemm_rows_tiles_ok(wt, n_in, &n_out, 1, b->tile_cnt != nullptr);
+}
+
+// n matrices of one type against the same rows: the rows prepared once, one
+// launch.  ws as in gemm_impl.
+int run_rows(krk_backend *b, void *const out[], const void *x, const void *const w[], int wt, const int64_t n_out[],
+             int64_t n_in, int n, int64_t rows, void *ws, size_t ws_bytes) {
+    const bool f16 = b->act == KRK_ACT_F16;
+    const int planes = !f16 && rows <= kRowsExact ? 2 : 1;
+    int64_t n_total = 0;
+    for (int m = 0; m < n; m++) n_total += n_out[m];
+    const size_t prep = krk::gemm_rows_prep_bytes(rows, n_in, planes, true);
+    const size_t need = prep + krk::gemm_rows_part_bytes(rows, n_total, n_in);
+    if (ws) {
+        if (need > ws_bytes)
+            return fail(b, KRK_ERR_NOMEM, "gemm rows need %zu bytes of scratch; the fixed scratch holds %zu", need,
+                        ws_bytes);
+    } else {
+        if (int s = ensure_ws(b, need)) return s;
+        ws = b->ws;
+    }
+    krk::RowsArgs a{};
+    hipError_t e = krk::gemm_rows_prep(wt, x, f16, n_in, rows, n_in, planes, true, nullptr, ws, a, b->stream);
+    if (e != hipSuccess) return hip_fail(b, e, "gemm rows");
+    for (int m = 0; m < n; m++) a.seg[m] = krk::RowsSeg{static_cast<const uint8_t *>(w[m]), out[m], n_out[m], 0};
+    a.part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) + prep);
+    a.cnt = b->tile_cnt;
+    a.n = n;
+    a.row_bytes = krk_dtype_row_bytes(wt, n_in);
+    a.rows = static_cast<int>(rows);
+    a.out_f16 = f16;
+    e = krk::gemm_rows(wt, a, b->stream);
+    return e == hipSuccess ? KRK_OK : hip_fail(b, e, "gemm rows");
+}
+
 // gemm with its scratch either in the handle's workspace (grown on demand,
 // ws == nullptr) or in a caller-fixed buffer of ws_bytes (never allocates)
 int gemm_impl(krk_backend *b, void *out, const void *x, const void *w, int wt, int64_t n_out, int64_t n_in,
@@ -314,6 +377,8 @@ int gemm_impl(krk_backend *b, void *out, const void *x, const void *w, int wt, i
     if (int s = make_current(b)) return s;
     const bool f16 = b->act == KRK_ACT_F16;
     const bool fixed = ws != nullptr;
+    if (rows_path(b, wt, n_out, n_in, rows, w))
+        return run_rows(b, &out, x, &w, wt, &n_out, n_in, 1, rows, ws, ws_bytes);
     if (rows <= 8 || b->path == KRK_PATH_EXACT) {
         krk::SegTable t = one_seg(w, x, out, wt, n_out, n_in, rows, krk::SEG_PLAIN, nullptr);
         if (rows > 1 && rows <= 8) {
@@ -418,7 +483,12 @@ int krk_gemm_group(krk_backend *b, void *const out[], const void *x, const void 
     const int nseg = n_mat - (silu ? 1 : 0);
     if (rows != 1 || !uniform || nseg > krk::kMaxSegs) {
         // the default Backend::gemm_group: one gemm per matrix, activation
-        // left to the caller
+        // left to the caller (rows of one type and one x: in one launch)
+        bool one = uniform && n_mat <= krk::kMaxSegs;
+        for (int m = 0; m < n_mat && one; m++)
+            one = (!xs || xs[m] == xs[0]) && rows_path(b, t0, n_out[m], n_in, rows, w[m]);
+        one = one && krk::gemm_rows_tiles_ok(t0, n_in, n_out, n_mat, b->tile_cnt != nullptr);
+        if (one) return run_rows(b, out, xs ? xs[0] : x, w, t0, n_out, n_in, n_mat, rows, nullptr, 0);
         for (int m = 0; m < n_mat; m++)
             if (int s = krk_gemm(b, out[m], xs ? xs[m] : x, w[m], wts ? wts[m] : wt, n_out[m], n_in,
                                  rows))
@@ -598,7 +668,7 @@ int krk_moe_dispatch(krk_backend *b, const void *table, int layer, int n_expert,
     a.rb_gate = e0.row_bytes[0]; a.rb_up = e0.row_bytes[1]; a.rb_down = e0.row_bytes[2];
     a.aligned16 = aligned;
     a.mfma = b->path != KRK_PATH_EXACT;
-    if (int s = ensure_ws(b, krk::moe_workspace(n_tok, k, n_expert, n_embd, n_ff))) return s;
+    if (int s = ensure_ws(b, krk::moe_workspace(a))) return s;
     const hipError_t he = krk::moe_dispatch(a, b->ws, b->ws_bytes, b->stream);
     return he == hipSuccess ? KRK_OK : hip_fail(b, he, "moe_dispatch");
 }

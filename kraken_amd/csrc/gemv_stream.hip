@@ -1,5 +1,5 @@
 // gemv_stream.hip -- decode GEMV (one activation row; dense Q4_K also two to
-// four) for Q4_K, Q6_K, Q4_0 and Q8_0 weights with every byte of a
+// five) for Q4_K, Q6_K, Q4_0 and Q8_0 weights with every byte of a
 // workgroup's tile requested in its first instructions, and the routed
 // expert modes of the MoE dispatch built on it.
 //
@@ -52,8 +52,8 @@ constexpr int kTabPad = 768, kTabEx = 784, kTabRows = 848;
 __host__ __device__ constexpr int tab_stride(int xr) { return xr > 1 ? kTabRows : kTab; }
 
 constexpr int kMaxWaves = 16;
-constexpr int kStreamRows = 8;   // dense Q4_K launches of up to this many activation rows
-constexpr int kStreamRowsWide = 4;   // ... of slices wider than two blocks
+constexpr int kStreamRows = 5;   // dense Q4_K launches of up to this many activation rows (more: gemm_rows.hip)
+constexpr int kStreamRowsWide = 3;   // ... of slices wider than two blocks
 constexpr size_t kLdsMax = 163840;   // LDS per workgroup on gfx950 (160 KB)
 
 __device__ __forceinline__ v4i lds_v4i(const uint8_t *p) { return *reinterpret_cast<const v4i *>(p); }
@@ -178,11 +178,10 @@ __global__ void __launch_bounds__(64) stream_xtab_kernel(const XT *__restrict__ 
 template <int DT, typename XT, typename OT, int NBW, int TR, int NWMAX, bool NWEXACT, int MOE = 0, int LA = 8,
           int XR = 1, bool LT = false>
 // (the second bound is waves per SIMD: four for the expert-major runs and
-// for six to eight rows, whose registers would otherwise leave one
-// workgroup per CU)
+// for five rows, whose registers would otherwise leave one workgroup per CU)
 __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8) ? 4 : 1)
     gemv_stream_kernel(SegTable t) {
-    // XR: activation rows (dense Q4_K launches of 2..4 rows): every row's
+    // XR: activation rows (dense Q4_K launches of 2..5 rows): every row's
     // activations load before the weights, one digit table per row, each
     // weight group decoded once and multiplied against every row
     static_assert(XR == 1 || (MOE == 0 && DT == DT_Q4_K), "several rows: dense Q4_K");
@@ -268,21 +267,16 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     // 8 (l & 3) .. + 7 of the slice's sub-block 16 p + l / 4
     // the loads issue at raised wave priority, so a wave that is still
     // issuing wins the vector-memory port over one that is already decoding
-    // rows per pass: six to eight rows run in passes of four, their digit
-    // tables rebuilt in the same (wave-private) LDS while the weights stay
-    // in registers, so two workgroups still fit a CU
-    constexpr int XP = XR > 5 ? 4 : XR;
-    float xvr[PAD ? 1 : XP][NPASS][8];
-    // (several rows: the pass's table slices, NBW 848-byte blocks per row,
+    float xvr[PAD ? 1 : XR][NPASS][8];
+    // (several rows: the table slices, NBW 848-byte blocks per row,
     // 16 bytes a lane per piece; copied from the call's precomputed tables)
     constexpr int PQ = PAD ? (NBW * (kTabRows / 16) + 63) / 64 : 1;
-    u32x4 tv[PAD ? XP : 1][PQ];
+    u32x4 tv[PAD ? XR : 1][PQ];
     const int nbp = PAD ? nw * NBW : 0;
-    auto load_tabs = [&](int r0, int r1) {
+    auto load_tabs = [&]() {
 #pragma unroll
-        for (int r = 0; r < XP; r++) {
-            if (r0 + r >= r1) break;
-            const uint8_t *src = t.xtab + (static_cast<int64_t>(r0 + r) * nbp + kb0) * kTabRows;
+        for (int r = 0; r < XR; r++) {
+            const uint8_t *src = t.xtab + (static_cast<int64_t>(r) * nbp + kb0) * kTabRows;
 #pragma unroll
             for (int j = 0; j < PQ; j++) {
                 const int q = 64 * j + lane;
@@ -305,11 +299,11 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     auto load_xrow = [&](const XT *xr) { load_xrow_to(xr, xvr[0]); };
     __builtin_amdgcn_s_setprio(3);
     if constexpr (PAD) {
-        load_tabs(0, XP);
+        load_tabs();
     } else {
         load_xrow(row_x(pb));
 #pragma unroll
-        for (int xr = 1; xr < XP; xr++) load_xrow_to(x + xr * t.x_stride, xvr[xr]);
+        for (int xr = 1; xr < XR; xr++) load_xrow_to(x + xr * t.x_stride, xvr[xr]);
     }
     // ---- then every weight byte of the wave's slice of the tile: group i =
     // (row group rg, block b), lane (c16, gq) takes of row rg * 16 + c16:
@@ -431,15 +425,15 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     // for Q6_K the exact integer sums of X over each 16-value half (int bits)
     // (several rows: the LDS holds XR times the tables, {2^-e, sum x}
     // arrays and partial sums, row by row)
-    // layout: XP table slots, then the XR rows' partial sums, then (LT) the
+    // layout: XR table slots, then the XR rows' partial sums, then (LT) the
     // slice buffers
     const int tstride = PAD ? nw * NBW * KT : nw * (NBW * KT + 2 * NBW * 8 * static_cast<int>(sizeof(float2)));
-    const int rstride = XP * tstride + XR * 32 * nw * 4;
+    const int rstride = XR * (tstride + 32 * nw * 4);
     auto tab_of = [&](int sl) { return lds + sl * tstride + wv * (NBW * KT); };
     auto ex_of = [&](int sl) {
         return reinterpret_cast<float2 *>(lds + sl * tstride + nw * (NBW * KT)) + wv * (NBW * 8);
     };
-    auto red_of = [&](int xr) { return reinterpret_cast<float *>(lds + XP * tstride + xr * 32 * nw * 4); };
+    auto red_of = [&](int xr) { return reinterpret_cast<float *>(lds + XR * tstride + xr * 32 * nw * 4); };
     // {2^-e, sum x} of block b of table slot sl
     auto ex_blk = [&](int sl, int b) -> const float2 * {
         if constexpr (PAD) return reinterpret_cast<const float2 *>(tab_of(sl) + b * KT + kTabEx);
@@ -471,26 +465,10 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     for (int xr = 0; xr < (XR > 1 ? XR - 1 : 1); xr++)
 #pragma unroll
         for (int rg = 0; rg < RG; rg++) accx[xr][rg] = 0.0f;
-#pragma unroll
-    for (int p0 = 0; p0 < XR; p0 += XP) {
-    const int pend = p0 + XP < XR ? p0 + XP : XR;
-    // (a later pass's activations: L2-resident rows, loaded once the
-    // previous pass has released their registers)
-    if (p0 > 0) {
-        if constexpr (PAD) {
-            load_tabs(p0, pend);
-        } else {
-#pragma unroll
-            for (int xr = p0; xr < pend; xr++) load_xrow_to(x + xr * t.x_stride, xvr[xr - p0]);
-        }
-    }
     if constexpr (PAD) {
-        // the pass's rows: their slices into the wave's table slots (this
-        // wave's reads of the previous pass completed in order before these
-        // writes)
+        // the rows' slices into the wave's table slots
 #pragma unroll
-        for (int r = 0; r < XP; r++) {
-            if (p0 + r >= pend) break;
+        for (int r = 0; r < XR; r++) {
 #pragma unroll
             for (int j = 0; j < PQ; j++) {
                 const int q = 64 * j + lane;
@@ -499,13 +477,13 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
         }
     } else {
 #pragma unroll
-    for (int xr = p0; xr < pend; xr++) {
-    uint8_t *tab = tab_of(xr - p0);
-    float2 *ex = ex_of(xr - p0);
+    for (int xr = 0; xr < XR; xr++) {
+    uint8_t *tab = tab_of(xr);
+    float2 *ex = ex_of(xr);
 #pragma unroll
     for (int p = 0; p < NPASS; p++) {
         const int sbw = p * 16 + (lane >> 2);
-        const float *v = xvr[xr - p0][p];
+        const float *v = xvr[xr][p];
         float amax = 0.0f, sum = 0.0f;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -614,7 +592,7 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     int lt_put = 0;   // instructions written to the buffer so far
 #pragma unroll
     for (int i = 0; i < NL; i++) {
-        if (!LT && i + LA < NL && pr == pb && p0 == 0) issue(i + LA);
+        if (!LT && i + LA < NL && pr == pb) issue(i + LA);
         __builtin_amdgcn_sched_barrier(0);
         const int rg = i / NBW, b = i - (i / NBW) * NBW;
         if constexpr (LT) {
@@ -902,17 +880,16 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
             a = __builtin_fmaf(-dmin * m1, e1.y, a);
             return a;
         };
-        if (p0 == 0) acc[rg] = row_dot(A0l, A1l, A0h, A1h, ex0, ex1, acc[rg]);
+        acc[rg] = row_dot(A0l, A1l, A0h, A1h, ex0, ex1, acc[rg]);
 #pragma unroll
-        for (int xr = p0 > 1 ? p0 : 1; xr < pend; xr++) {
-            const float2 *ey = ex_blk(xr - p0, b);
+        for (int xr = 1; xr < XR; xr++) {
+            const float2 *ey = ex_blk(xr, b);
             v4i a0l, a1l, a0h, a1h;
-            a_ops(tab_of(xr - p0) + b * KT, a0l, a1l, a0h, a1h);
+            a_ops(tab_of(xr) + b * KT, a0l, a1l, a0h, a1h);
             accx[xr - 1][rg] = row_dot(a0l, a1l, a0h, a1h, ey[gq], ey[4 + gq], accx[xr - 1][rg]);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    }   // passes of activation rows
 
     // ---- the waves' partial sums -> LDS [row][wave]; one thread per output
     // row adds them in wave order
@@ -967,9 +944,8 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
 
 
 size_t stream_lds(int nw, int nbw, int xr = 1) {
-    const size_t xp = xr > 5 ? 4 : xr;   // table slots: rows per pass
     const size_t per = xr > 1 ? kTabRows : kTab + 2 * 8 * sizeof(float2);
-    return xp * nw * nbw * per + xr * 32 * static_cast<size_t>(nw) * sizeof(float);
+    return xr * nw * nbw * per + xr * 32 * static_cast<size_t>(nw) * sizeof(float);
 }
 // the load-transpose slice buffers of a launch
 size_t stream_lt_lds(int nw, int nbw, int tr, int pb = 9) {
@@ -1103,8 +1079,8 @@ bool gemv_stream_ok(int dt, const SegTable &t) {
     int64_t rows = 0;
     for (int i = 0; i < t.n; i++) rows += t.seg[i].n_out;
     const int nw = (t.n_in / 256 + nbw - 1) / nbw;
-    // (several rows: their digit tables within the 160 KB of LDS; five and
-    // more rows on two-block slices)
+    // (several rows: their digit tables within the 160 KB of LDS; four and
+    // five rows on two-block slices)
     if (t.rows > 1 && (!t.xtab || stream_lds(nw, nbw, static_cast<int>(t.rows)) > kLdsMax ||
                        (t.rows > kStreamRowsWide && nbw != 2)))
         return false;
@@ -1220,9 +1196,7 @@ hipError_t gemv_stream(int dt, bool act_f16, const SegTable &t0, hipStream_t st)
     const int64_t cap = static_cast<int64_t>(device_cus()) * per_cu;
     int tr = 16;
     int64_t best = INT64_MAX;
-    // (six to eight rows: 16-row tiles; taller ones spill 25-27 registers at
-    // the four waves per SIMD these rows run at, 27-40 us against 20 at 8 rows)
-    for (int c = has_pair ? 32 : 16; c <= (nbw > 2 || t.rows > 5 ? 16 : 32); c += 4) {
+    for (int c = has_pair ? 32 : 16; c <= (nbw > 2 ? 16 : 32); c += 4) {
         int64_t tiles = 0;
         for (int i = 0; i < t.n; i++) {
             const int rows_t = t.seg[i].kind == SEG_SILU ? 16 : c;
@@ -1274,19 +1248,10 @@ hipError_t gemv_stream(int dt, bool act_f16, const SegTable &t0, hipStream_t st)
         case 4:
             return act_f16 ? launch_nbw<DT_Q4_K, _Float16, _Float16, 4>(nbw, t, tr, width, nw, st)
                            : launch_nbw<DT_Q4_K, float, float, 4>(nbw, t, tr, width, nw, st);
-        // five to eight rows: two-block slices only (gemv_stream_ok)
+        // five rows: two-block slices only (gemv_stream_ok)
         case 5:
             return act_f16 ? launch_tr<DT_Q4_K, _Float16, _Float16, 2, 5>(t, tr, width, nw, st)
                            : launch_tr<DT_Q4_K, float, float, 2, 5>(t, tr, width, nw, st);
-        case 6:
-            return act_f16 ? launch_tr<DT_Q4_K, _Float16, _Float16, 2, 6>(t, tr, width, nw, st)
-                           : launch_tr<DT_Q4_K, float, float, 2, 6>(t, tr, width, nw, st);
-        case 7:
-            return act_f16 ? launch_tr<DT_Q4_K, _Float16, _Float16, 2, 7>(t, tr, width, nw, st)
-                           : launch_tr<DT_Q4_K, float, float, 2, 7>(t, tr, width, nw, st);
-        case 8:
-            return act_f16 ? launch_tr<DT_Q4_K, _Float16, _Float16, 2, 8>(t, tr, width, nw, st)
-                           : launch_tr<DT_Q4_K, float, float, 2, 8>(t, tr, width, nw, st);
         default: break;
     }
     return act_f16 ? launch_nbw<DT_Q4_K, _Float16, _Float16>(nbw, t, tr, width, nw, st)

@@ -77,12 +77,57 @@ struct SegTable {
     // row em_tok[p] (row p when em_tok is null), outputs seg[0].out row p.
     const EmRun *em_runs;
     const int32_t *em_n_act;
-    // Dense launches of 2..8 activation rows on the streaming kernel: device
+    // Dense launches of 2..5 activation rows on the streaming kernel: device
     // scratch of gemv_stream_xtab_bytes(rows, n_in) for the rows' digit
     // tables, built once per call (nullable: then those launches take the
     // other kernels)
     uint8_t *xtab;
 };
+
+// Several activation rows against weights streamed once (gemm_rows.hip):
+// dense segments, or (runs) the active experts' banks over their plan
+// positions.  xp / inv / planes / nb come from gemm_rows_prep.
+struct RowsSeg {
+    const uint8_t *w;
+    void *out;
+    int64_t n_out;
+    int64_t col;             // first column of the segment in the partials (set by gemm_rows)
+};
+struct RowsArgs {
+    RowsSeg seg[kMaxSegs];
+    int n;
+    int64_t row_bytes;
+    int nb;                  // 256-value blocks of a weight row
+    const uint8_t *xp;       // prepared activation rows
+    const float *inv;        // and the scale each one's results take
+    int planes;              // 1: f16 rows (or f32 rounded to f16); 2: f32 rows, hi + lo
+    int rows;                // dense: activation rows
+    bool out_f16;            // dense outputs in f16
+    // dense, K of more than 16 blocks: gemm_rows_part_bytes of scratch for the
+    // K ranges' partials, and zeroed tile counters (left zero)
+    float *part;
+    unsigned *cnt;
+    int64_t part_n;          // columns of the partials and blocks of a K range (set by gemm_rows)
+    int range;
+    // routed: run y = grid row y while y < *n_act: its plan positions'
+    // activations are prepared rows tok[p] (p when tok is null); outputs f32
+    // rows p of seg[0].out.  pair: gate/up banks, silu(gate) * up (act_f16:
+    // with the f16 roundings of the f16 path); else the down bank.
+    const EmRun *runs;
+    const int32_t *n_act;
+    const int32_t *tok;
+    int max_runs;
+    bool pair, act_f16;
+};
+// whether a dense launch's tiles fit the K ranges' counters (or needs none)
+bool gemm_rows_tiles_ok(int dt, int64_t n_in, const int64_t n_out[], int n, bool counters);
+bool gemm_rows_ok(int dt, int64_t n_in, const void *w, int64_t row_bytes);
+size_t gemm_rows_prep_bytes(int64_t rows, int64_t n_in, int planes, bool dense);
+// prepares `rows` rows (of them the first *n_rows when given) into ws
+hipError_t gemm_rows_prep(int dt, const void *x, bool x_f16, int64_t x_stride, int64_t rows, int64_t n_in, int planes,
+                          bool dense, const int32_t *n_rows, void *ws, RowsArgs &a, hipStream_t st);
+size_t gemm_rows_part_bytes(int64_t rows, int64_t n_total, int64_t n_in);
+hipError_t gemm_rows(int dt, const RowsArgs &a, hipStream_t st);
 
 hipError_t gemv_segments(int dt, bool act_f16, const SegTable &t, hipStream_t st);
 // Q4_K, Q6_K, Q4_0 and Q8_0, one activation row (or the rows of expert-major
@@ -182,7 +227,7 @@ struct MoeArgs {
     bool aligned16;      // every bank's rows start 16-byte aligned
     bool mfma;           // the gemm path allows f16 MFMA products (not KRK_PATH_EXACT)
 };
-size_t moe_workspace(int64_t n_tok, int k, int n_expert, int64_t n_embd, int64_t n_ff);
+size_t moe_workspace(const MoeArgs &a);
 hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t st);
 
 }  // namespace krk

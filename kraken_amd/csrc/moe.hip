@@ -67,6 +67,7 @@ struct MoeWs {
     float *rscale;      // [P]            f16 activations: each mid row's power-of-two scale
     EmRun *runs;        // [n_expert]     active experts' banks and plan ranges
     _Float16 *xg;       // [P, n_embd]    grouped GEMM: the tokens' activation rows, f16
+    uint8_t *prep;      // rows kernel: the tokens' prepared rows, then the mid rows'
 };
 
 static size_t al(size_t v) { return (v + 255) & ~size_t(255); }
@@ -86,13 +87,31 @@ static MoeWs carve(void *ws, int64_t P, int ne, int64_t n_embd, int64_t n_ff) {
     w.midf = reinterpret_cast<_Float16 *>(p); p += al(P * n_ff * 2);
     w.rscale = reinterpret_cast<float *>(p); p += al(P * 4);
     w.runs = reinterpret_cast<EmRun *>(p); p += al(ne * sizeof(EmRun));
-    w.xg = reinterpret_cast<_Float16 *>(p);
+    w.xg = reinterpret_cast<_Float16 *>(p); p += al(P * n_embd * 2);
+    w.prep = p;
     return w;
 }
 
-size_t moe_workspace(int64_t n_tok, int k, int n_expert, int64_t n_embd, int64_t n_ff) {
+// Calls whose experts run on the rows kernel (gemm_rows.hip): exact products
+// over each active expert's tokens, its banks streamed once.  Layers of one
+// gate/up type and one down type among Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0;
+// kRowsMoeF32: the f32 batches it takes (below, with the figures).
+static bool moe_rows(const MoeArgs &a) {
+    if (a.wt < 0 || a.rb_gate != a.rb_up || !a.aligned16 || a.n_embd > 8192) return false;
+    if (!gemm_rows_ok(a.wt, a.n_embd, nullptr, a.rb_gate) || !gemm_rows_ok(a.wt_down, a.n_ff, nullptr, a.rb_down))
+        return false;
+    return a.act_f16;
+}
+
+size_t moe_workspace(const MoeArgs &a) {
+    const int64_t n_tok = a.n_tok, n_embd = a.n_embd, n_ff = a.n_ff;
+    const int k = a.k, n_expert = a.n_expert;
     const int64_t P = n_tok * k;
-    return al((n_expert + 1) * 4) + al(n_expert * 4) + al(4) + 2 * al(P * 4) +
+    const int planes = a.act_f16 ? 1 : 2;
+    const size_t prep = moe_rows(a) ? al(gemm_rows_prep_bytes(n_tok, n_embd, planes, false)) +
+                                          al(gemm_rows_prep_bytes(P, n_ff, planes, false))
+                                    : 0;
+    return prep + al((n_expert + 1) * 4) + al(n_expert * 4) + al(4) + 2 * al(P * 4) +
            al(P * n_ff * 4) + al(P * n_embd * 4) + al(P * 16) + al(4) + al(P * n_ff * 2) + al(P * 4) +
            al(n_expert * sizeof(EmRun)) + al(P * n_embd * 2);
 }
@@ -537,7 +556,7 @@ constexpr int64_t kMoeGemmTokens = 32;
 
 hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t st) {
     const int64_t P = a.n_tok * a.k;
-    if (ws_bytes < moe_workspace(a.n_tok, a.k, a.n_expert, a.n_embd, a.n_ff)) return hipErrorInvalidValue;
+    if (ws_bytes < moe_workspace(a)) return hipErrorInvalidValue;
     if (a.n_expert > 1024 || a.k > 64) return hipErrorInvalidValue;
     MoeWs w = carve(ws, P, a.n_expert, a.n_embd, a.n_ff);
     const krk_moe_entry *tab = static_cast<const krk_moe_entry *>(a.table) +
@@ -664,6 +683,50 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
         const dim3 rgrid(static_cast<unsigned>((a.n_embd + 255) / 256), static_cast<unsigned>(a.n_tok));
         hipLaunchKernelGGL((moe_reduce_kernel<float>), rgrid, dim3(256), 0, st, a.ids, a.wts, a.k,
                            a.n_embd, w, static_cast<float *>(a.out));
+        return hipGetLastError();
+    }
+    if (moe_rows(a)) {
+        // plan; the tokens' rows prepared; gate/up of every active expert into
+        // mid; (f16: each mid row scaled and rounded) the mid rows prepared;
+        // down into part; the ordered reduce
+        const int planes = a.act_f16 ? 1 : 2;
+        hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(256), 0, st, a.ids, P, a.k, a.n_expert, w, tab,
+                           kItemRows);
+        RowsArgs r{};
+        r.n = 1;
+        r.runs = w.runs;
+        r.n_act = w.n_act;
+        r.max_runs = static_cast<int>(P < a.n_expert ? P : a.n_expert);
+        r.act_f16 = a.act_f16;
+        hipError_t e = gemm_rows_prep(a.wt, a.xn, a.act_f16, a.n_embd, a.n_tok, a.n_embd, planes, false, nullptr, w.prep,
+                                      r, st);
+        if (e != hipSuccess) return e;
+        r.tok = w.plan_tok;
+        r.row_bytes = a.rb_gate;
+        r.pair = true;
+        r.seg[0] = RowsSeg{nullptr, w.mid, a.n_ff, 0};
+        e = gemm_rows(a.wt, r, st);
+        if (e != hipSuccess) return e;
+        uint8_t *prep2 = w.prep + al(gemm_rows_prep_bytes(a.n_tok, a.n_embd, planes, false));
+        if (a.act_f16)
+            hipLaunchKernelGGL(moe_scale_kernel, dim3(static_cast<unsigned>(P)), dim3(256), 0, st, a.n_ff,
+                               a.n_expert, w);
+        e = gemm_rows_prep(a.wt_down, a.act_f16 ? static_cast<const void *>(w.midf) : w.mid, a.act_f16, a.n_ff, P, a.n_ff,
+                           planes, false, w.off + a.n_expert, prep2, r, st);
+        if (e != hipSuccess) return e;
+        r.tok = nullptr;
+        r.row_bytes = a.rb_down;
+        r.pair = false;
+        r.seg[0] = RowsSeg{nullptr, w.part, a.n_embd, 0};
+        e = gemm_rows(a.wt_down, r, st);
+        if (e != hipSuccess) return e;
+        const dim3 rgrid(static_cast<unsigned>((a.n_embd + 255) / 256), static_cast<unsigned>(a.n_tok));
+        if (a.act_f16)
+            hipLaunchKernelGGL(moe_reduce_f16_kernel, rgrid, dim3(256), 0, st, a.wts, a.k, a.n_embd, w,
+                               static_cast<_Float16 *>(a.out));
+        else
+            hipLaunchKernelGGL((moe_reduce_kernel<float>), rgrid, dim3(256), 0, st, a.ids, a.wts, a.k,
+                               a.n_embd, w, static_cast<float *>(a.out));
         return hipGetLastError();
     }
     if (on_stream && a.n_tok >= 2) {
