@@ -11,8 +11,8 @@
 // ramp and tail (the preparation's launch, the first loads' latency, the
 // waves' sums).  Measured, Q4_K f16 rows: 4096 -> 14336 8 rows 19.4 -> 16.0 us,
 // 14336 -> 4096 8 rows 80.9 -> 20.8 us (6.7 us of HBM time each); the f16
-// expert layer (128 experts, 4096 / 1536, top 8) 160 tokens 9797 -> 556 us,
-// one token 233 -> 61 us.  What the layout buys:
+// expert layer (128 experts, 4096 / 1536, top 8) 160 tokens 9797 -> 435 us,
+// one token 233 -> 65 us.  What the layout buys:
 //   * A workgroup owns 16 or 32 weight rows over all of K; its waves split K
 //     into contiguous slices of NBW 256-value blocks, and a wave requests
 //     every weight byte of its slice before any arithmetic, so no barrier or
@@ -489,132 +489,103 @@ __global__ void __launch_bounds__(256) rows_prep_kernel(const XT *__restrict__ x
     }
 }
 
-// One workgroup: weight rows [n0, n0 + 16 RG) of a segment (gate/up pairs:
-// 8 RG gate rows and the same up rows) over the blocks of K range blockIdx.z,
-// against all of its activation rows, 16 prepared rows a pass.  Two planes:
-// prepared rows 0..7 of a pass are the hi planes of eight rows, 8..15 their lo
-// planes.
-// NWX: exactly NWMAX waves, which lets the final sums' reads all be in flight
-template <int DT, int NBW, int RG, int NWMAX, bool NWX, bool DENSE>
+// One output's sums of the waves, in wave order (at: wave 0's, `wave` floats
+// apart; two planes: the lo plane's row lies `lo` floats on).  NWX: exactly
+// NWMAX waves, which lets the reads all be in flight.
+template <int NWMAX, bool NWX>
+__device__ __forceinline__ float wave_sums(const float *at, int wave, int lo, int nw, int planes) {
+    float v = 0.0f;
+    if (planes == 2) {
+#pragma unroll
+        for (int q = 0; q < NWMAX; q++)
+            if (NWX || q < nw) v += at[q * wave] + at[q * wave + lo];
+    } else {
+#pragma unroll
+        for (int q = 0; q < NWMAX; q++)
+            if (NWX || q < nw) v += at[q * wave];
+    }
+    return v;
+}
+
+// Dense.  One workgroup: weight rows [n0, n0 + 16 RG) of a segment over the
+// blocks of K range blockIdx.z, one a wave, against all activation rows, 16
+// prepared rows a pass.
+template <int DT, int RG, int NWMAX, bool NWX>
 __global__ void __launch_bounds__(64 * NWMAX) __attribute__((amdgpu_waves_per_eu(4))) rows_kernel(RowsArgs a) {
     extern __shared__ __align__(16) float red[];
     constexpr int S = 16 * RG + 4;          // red row stride: the four lane rows' stores spread over the banks
-    using At = PrepAt<DENSE>;
-    constexpr int H = RG / 2;               // row groups of each half of a pair
+    using At = PrepAt<true>;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nw = NWX ? NWMAX : static_cast<int>(blockDim.x) >> 6;
     const int j = lane & 15, g = lane >> 4;
     const int kz = static_cast<int>(blockIdx.z) * a.range;   // this K range's first block
     const int kend = kz + a.range < a.nb ? kz + a.range : a.nb;
-    const int kb0 = kz + wv * NBW;
-    const uint8_t *w, *w2;
-    void *out;
-    int64_t n_out;
-    int p_begin = 0, p_end = a.rows;
-    const bool pair = a.pair;
-    if constexpr (!DENSE) {
-        const EmRun &run = a.runs[blockIdx.y];
-        if (static_cast<int>(blockIdx.y) >= *a.n_act) return;
-        p_begin = run.pb;
-        p_end = run.pe;
-        w = static_cast<const uint8_t *>(run.w[pair ? 0 : 2]);
-        w2 = static_cast<const uint8_t *>(run.w[1]);
-        out = a.seg[0].out;
-        n_out = a.seg[0].n_out;
-    } else {
-        const RowsSeg &sg = a.seg[blockIdx.y];
-        w = w2 = sg.w;
-        out = sg.out;
-        n_out = sg.n_out;
-    }
-    const int rows_sh = (RG == 4 ? 6 : RG == 2 ? 5 : 4) - (pair ? 1 : 0), rows_t = 1 << rows_sh;
+    const int blk = kz + wv;
+    const bool live = blk < kend;           // (a range shorter than the others leaves its last wave idle)
+    const RowsSeg &sg = a.seg[blockIdx.y];
+    void *out = sg.out;
+    const int64_t n_out = sg.n_out;
+    constexpr int rows_sh = RG == 4 ? 6 : RG == 2 ? 5 : 4, rows_t = 1 << rows_sh;
     const int64_t n0 = static_cast<int64_t>(blockIdx.x) * rows_t;
     if (n0 >= n_out) return;                // a segment shorter than the grid's width
     const int per = a.planes == 2 ? 8 : 16;             // rows a pass
-    const int nbl = kend - kb0 < NBW ? kend - kb0 : NBW;    // blocks of this wave's slice (none: an idle last wave)
 
-    // the pass's prepared rows
-    gbyte *xrow = nullptr;
-    auto point = [&](int p0) {
-        int64_t r;
-        if constexpr (DENSE) {
-            // (sixteen prepared rows a pass; those past the last hold whatever
-            // was there, and their results go nowhere)
-            r = 16 * (p0 / per) + j;
-        } else {
-            int p = p0 + (a.planes == 2 ? (j & 7) : j);
-            p = p < p_end ? p : p0;         // rows past the end re-read the pass's first
-            const int64_t t = a.tok ? a.tok[p] : p;
-            r = a.planes == 2 ? 2 * t + (j >> 3) : t;
-        }
-        xrow = to_global(a.xp) + At::row(r, a.nb) + static_cast<int64_t>(kb0) * At::kBlock + At::kPiece * g;
-    };
-    // one block's activation fragments: once a pair is multiplied, its
-    // registers take the same pair of the next block, or of the next pass
+    // the pass's prepared rows (sixteen; those past the last hold whatever was
+    // there, and their results go nowhere).  Once a pair of sub-blocks is
+    // multiplied, its registers take the same pair of the next pass.
+    gbyte *xrow = to_global(a.xp) + At::row(j, a.nb) + static_cast<int64_t>(blk) * At::kBlock + At::kPiece * g;
     u32x4 xa[4][2], xs = {0u, 0u, 0u, 0u};
-    auto load_pair = [&](int p, int b) {
+    auto load_pair = [&](int p) {
 #pragma unroll
-        for (int s = 0; s < 2; s++) xa[p][s] = ld128(xrow + b * At::kBlock + At::kPart * (2 * p + s));
+        for (int s = 0; s < 2; s++) xa[p][s] = ld128(xrow + At::kPart * (2 * p + s));
     };
-    auto load_sums = [&](int b) {
-        if constexpr (has_min(DT)) xs = ld128(xrow + b * At::kBlock + At::kPart * 8);
+    auto load_sums = [&]() {
+        if constexpr (has_min(DT)) xs = ld128(xrow + At::kPart * 8);
     };
     const Masks masks;
-    RowBlk<DT> wr[NBW][RG];
-    if (nbl > 0) {
-        point(p_begin);
+    RowBlk<DT> wr[RG];
+    if (live) {
 #pragma unroll
-        for (int p = 0; p < 4; p++) load_pair(p, 0);
-        load_sums(0);
-        // every weight byte of the wave's slice (a ragged last slice re-reads
-        // its last block, unused)
+        for (int p = 0; p < 4; p++) load_pair(p);
+        load_sums();
+        // every weight byte of the wave's block of the tile
 #pragma unroll
-        for (int b = 0; b < NBW; b++)
-#pragma unroll
-            for (int r = 0; r < RG; r++) {
-                int64_t n = n0 + 16 * (pair && H && r >= H ? r - H : r) + j;
-                n = n < n_out ? n : n_out - 1;
-                wr[b][r].fetch(to_global((pair && r >= H ? w2 : w) + n * a.row_bytes) +
-                                   static_cast<int64_t>(kb0 + (b < nbl ? b : nbl - 1)) * RowBlk<DT>::BB,
-                               g);
-            }
+        for (int r = 0; r < RG; r++) {
+            int64_t n = n0 + 16 * r + j;
+            n = n < n_out ? n : n_out - 1;
+            wr[r].fetch(to_global(sg.w + n * a.row_bytes) + static_cast<int64_t>(blk) * RowBlk<DT>::BB, g);
+        }
     }
 
     const int64_t prow = static_cast<int64_t>(a.rows) * a.part_n;   // floats of one K range's partials
-    for (int p0 = p_begin; p0 < p_end; p0 += per) {
-        const bool more = p0 + per < p_end;
+    for (int p0 = 0; p0 < a.rows; p0 += per) {
+        const bool more = p0 + per < a.rows;
         floatx4 acc[RG];
 #pragma unroll
         for (int r = 0; r < RG; r++) acc[r] = KRK_ZERO4;
-#pragma unroll
-        for (int b = 0; b < NBW; b++) {
-            if (b >= nbl) break;            // wave-uniform
-            // where the registers of a multiplied pair refill from
-            const bool last = b + 1 >= nbl;
-            if (last && more) point(p0 + per);
-            const int nb = last ? 0 : b + 1;
-            const bool refill = !last || more;
+        if (live) {
+            if (more) xrow += At::stride(a.nb);
             // row group by row group, in the order they were requested: a
             // group is multiplied while the next ones are still on their way
             // (the scheduling barriers keep the pairs' operands from all being
             // built at once, which would not fit the registers)
 #pragma unroll
             for (int r = 0; r < RG; r++) {
-                if (p0 == p_begin) wr[b][r].settle();
-                wr[b][r].hold();
+                if (p0 == 0) wr[r].settle();
+                wr[r].hold();
                 floatx4 t = KRK_ZERO4;
-#define KRK_PAIR(P)                                    \
-    __builtin_amdgcn_sched_barrier(0);                 \
-    wr[b][r].template pair<P>(xa[P], masks, t, acc[r]);\
-    settle_acc(DT == DT_Q4_K || DT == DT_Q5_K ? t : acc[r]); \
-    if (r == RG - 1 && refill) load_pair(P, nb);       \
+#define KRK_PAIR(P)                                                   \
+    __builtin_amdgcn_sched_barrier(0);                                \
+    wr[r].template pair<P>(xa[P], masks, t, acc[r]);                  \
+    settle_acc(DT == DT_Q4_K || DT == DT_Q5_K ? t : acc[r]);          \
+    if (r == RG - 1 && more) load_pair(P);                            \
     __builtin_amdgcn_sched_barrier(0);
                 KRK_PAIR(0) KRK_PAIR(1) KRK_PAIR(2) KRK_PAIR(3)
 #undef KRK_PAIR
-                wr[b][r].finish(xs, masks, t, acc[r]);
+                wr[r].finish(xs, masks, t, acc[r]);
                 settle_acc(acc[r]);
-                if (r == RG - 1 && refill) load_sums(nb);
+                if (r == RG - 1 && more) load_sums();
             }
         }
         // lane (j, g): weight row j, activation rows 4g .. 4g + 3
@@ -623,55 +594,27 @@ __global__ void __launch_bounds__(64 * NWMAX) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
             for (int k = 0; k < 4; k++) red[(wv * 16 + 4 * g + k) * S + 16 * r + j] = acc[r][k];
         __syncthreads();
-        const int left = p_end - p0 < per ? p_end - p0 : per;
+        const int left = a.rows - p0 < per ? a.rows - p0 : per;
         for (int o = tid; o < left * rows_t; o += 64 * nw) {
             const int i = o >> rows_sh, c = o - (i << rows_sh), p = p0 + i;
             const int64_t n = n0 + c;
             if (n >= n_out) continue;
             // (requested before the sums, not after)
-            const float inv = a.inv[!DENSE && a.tok ? a.tok[p] : p];
-            // the waves' sums in order; a row's lo plane lies eight rows on
-            auto total = [&](int col) {
-                float v = 0.0f;
-                const float *at = red + i * S + col;
-                if (a.planes == 2) {
-#pragma unroll
-                    for (int q = 0; q < NWMAX; q++)
-                        if (NWX || q < nw) v += at[q * 16 * S] + at[(q * 16 + 8) * S];
-                } else {
-#pragma unroll
-                    for (int q = 0; q < NWMAX; q++)
-                        if (NWX || q < nw) v += at[q * 16 * S];
-                }
-                return v;
-            };
-            if (a.part) {   // (dense) this K range's partial
+            const float inv = a.inv[p];
+            const float v = wave_sums<NWMAX, NWX>(red + i * S + c, 16 * S, 8 * S, nw, a.planes);
+            if (a.part) {   // this K range's partial
                 __hip_atomic_store(a.part + blockIdx.z * prow + static_cast<int64_t>(p) * a.part_n +
                                        a.seg[blockIdx.y].col + n,
-                                   total(c), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                                   v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 continue;
             }
-            if (pair) {
-                float gt = total(c) * inv, up = total(16 * H + c) * inv;
-                if (a.act_f16) {
-                    // both dots rounded to f16 first, silu with the device
-                    // exponential (moe_table.hpp:250-253)
-                    gt = static_cast<float>(static_cast<_Float16>(gt));
-                    up = static_cast<float>(static_cast<_Float16>(up));
-                    static_cast<float *>(out)[p * n_out + n] = silu_f(gt) * up;
-                } else {
-                    static_cast<float *>(out)[p * n_out + n] = (gt / (1.0f + expf(-gt))) * up;
-                }
-            } else if (a.out_f16) {
-                static_cast<_Float16 *>(out)[p * n_out + n] = static_cast<_Float16>(total(c) * inv);
-            } else {
-                static_cast<float *>(out)[p * n_out + n] = total(c) * inv;
-            }
+            if (a.out_f16) static_cast<_Float16 *>(out)[p * n_out + n] = static_cast<_Float16>(v * inv);
+            else static_cast<float *>(out)[p * n_out + n] = v * inv;
         }
         __syncthreads();
     }
     if (!a.part) return;
-    // K ranges (dense): each workgroup's partials are complete before it
+    // K ranges: each workgroup's partials are complete before it
     // counts itself in the tile's counter; the last to arrive adds the ranges'
     // partials in range order, so the result does not depend on which one
     // that is, and clears the counter for the next call.  Partials and
@@ -701,17 +644,215 @@ __global__ void __launch_bounds__(64 * NWMAX) __attribute__((amdgpu_waves_per_eu
     if (tid == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int DT, int NBW, int RG, bool DENSE>
-hipError_t launch(const RowsArgs &a, dim3 grid, int nw, hipStream_t st) {
+// Routed.  Persistent workgroups over chunks of `ct` weight tiles of one active
+// expert (chunk c: run c / chunks per run), its waves splitting K into slices
+// of NBW blocks.  A tile is 16 RG weight rows (gate/up pairs: 8 RG gate rows
+// and the same up rows), multiplied with the expert's prepared rows, 16 a pass.
+// A row group's registers take the same group of the next tile as soon as its
+// last pass is multiplied, and the activations stay in registers while the
+// expert and its pass do (one-block slices), so the weights stream without a
+// pause: one workgroup per tile with everything requested up front left the
+// memory idle while it multiplied and summed (gate/up of 160 tokens, 906 MB:
+// 339 -> 269 us, down, 453 MB: 189 -> 140 us; the loads alone take 3/4 of it).  The waves' sums alternate between two LDS buffers, one barrier a
+// step; it is a bare one, so that the requests in flight stay so.
+template <int DT, int NBW, int RG, int NWMAX, bool NWX>
+__global__ void __launch_bounds__(64 * NWMAX) __attribute__((amdgpu_waves_per_eu(4)))
+    rows_routed_kernel(RowsArgs a, int tiles, int ct) {
+    extern __shared__ __align__(16) float red_lds[];
+    constexpr int S = 16 * RG + 4;
+    using At = PrepAt<false>;
+    constexpr int H = RG / 2;               // row groups of each half of a pair
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nw = NWX ? NWMAX : static_cast<int>(blockDim.x) >> 6;
+    const int j = lane & 15, g = lane >> 4;
+    const int kb0 = wv * NBW;
+    const int nbl = a.nb - kb0 < NBW ? a.nb - kb0 : NBW;    // blocks of this wave's slice (at least one)
+    const bool pair = a.pair;
+    const int rows_sh = (RG == 4 ? 6 : RG == 2 ? 5 : 4) - (pair ? 1 : 0), rows_t = 1 << rows_sh;
+    const int per = a.planes == 2 ? 8 : 16;                 // rows a pass
+    const int64_t n_out = a.seg[0].n_out;
+    float *out = static_cast<float *>(a.seg[0].out);
+    const int cpr = (tiles + ct - 1) / ct, chunks = *a.n_act * cpr;
+    int chunk = static_cast<int>(blockIdx.x);
+    if (chunk >= chunks) return;
+
+    struct Step {
+        const uint8_t *w, *w2;
+        int tile, tend, pb, pe, p0;
+    };
+    auto open = [&](int c) {
+        const int run = c / cpr;
+        const EmRun &r = a.runs[run];
+        Step s;
+        s.w = static_cast<const uint8_t *>(r.w[pair ? 0 : 2]);
+        s.w2 = static_cast<const uint8_t *>(r.w[1]);
+        s.tile = (c - run * cpr) * ct;
+        s.tend = s.tile + ct < tiles ? s.tile + ct : tiles;
+        s.pb = s.p0 = r.pb;
+        s.pe = r.pe;
+        return s;
+    };
+    gbyte *xrow = nullptr;
+    auto point = [&](const Step &s) {
+        int p = s.p0 + (a.planes == 2 ? (j & 7) : j);
+        p = p < s.pe ? p : s.p0;            // rows past the end re-read the pass's first
+        const int64_t t = a.tok ? a.tok[p] : p;
+        xrow = to_global(a.xp) + At::row(a.planes == 2 ? 2 * t + (j >> 3) : t, a.nb) +
+               static_cast<int64_t>(kb0) * At::kBlock + At::kPiece * g;
+    };
+    u32x4 xa[4][2], xs = {0u, 0u, 0u, 0u};
+    auto load_pair = [&](int p, int b) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) xa[p][s] = ld128(xrow + b * At::kBlock + At::kPart * (2 * p + s));
+    };
+    auto load_sums = [&](int b) {
+        if constexpr (has_min(DT)) xs = ld128(xrow + b * At::kBlock + At::kPart * 8);
+    };
+    const Masks masks;
+    RowBlk<DT> wr[NBW][RG];
+    // a uniform row base and a 32-bit lane offset (rows are shorter than 2^26
+    // bytes); rows past the bank's last re-read it, a ragged last slice its
+    // last block, unused
+    const uint32_t rb = static_cast<uint32_t>(a.row_bytes);
+    auto fetch = [&](const Step &s, int b, int r) {
+        int64_t n = static_cast<int64_t>(s.tile) * rows_t + 16 * (pair && H && r >= H ? r - H : r);
+        n = n < n_out ? n : n_out - 1;
+        const int lim = n_out - n < 16 ? static_cast<int>(n_out - n) - 1 : 15;
+        gbyte *base = to_global(pair && r >= H ? s.w2 : s.w) + n * a.row_bytes +
+                      static_cast<int64_t>(kb0 + (b < nbl ? b : nbl - 1)) * RowBlk<DT>::BB;
+        wr[b][r].fetch(base + static_cast<uint32_t>(j < lim ? j : lim) * rb, g);
+    };
+    Step cur = open(chunk);
+    point(cur);
+#pragma unroll
+    for (int p = 0; p < 4; p++) load_pair(p, 0);
+    load_sums(0);
+#pragma unroll
+    for (int b = 0; b < NBW; b++)
+#pragma unroll
+        for (int r = 0; r < RG; r++) fetch(cur, b, r);
+
+    for (int buf = 0;; buf ^= 1) {
+        // the next step: whether it brings another tile, other activations
+        Step nxt = cur;
+        bool wn = false, xn = true, end = false;
+        if (cur.p0 + per < cur.pe) {
+            nxt.p0 += per;
+        } else {
+            wn = true;
+            nxt.p0 = cur.pb;
+            if (++nxt.tile < cur.tend) {
+                xn = cur.pe - cur.pb > per;
+            } else {
+                chunk += static_cast<int>(gridDim.x);
+                end = chunk >= chunks;
+                if (!end) nxt = open(chunk);
+                wn = xn = !end;
+            }
+        }
+        const bool xr = !end && (xn || nbl > 1);
+        // this thread's first output's row scale, needed after the barrier
+        const int left = cur.pe - cur.p0 < per ? cur.pe - cur.p0 : per;
+        const int i0 = tid >> rows_sh;
+        const int t0 = i0 < left ? cur.p0 + i0 : cur.p0;
+        float inv = a.inv[a.tok ? a.tok[t0] : t0];
+        floatx4 acc[RG];
+#pragma unroll
+        for (int r = 0; r < RG; r++) acc[r] = KRK_ZERO4;
+#pragma unroll
+        for (int b = 0; b < NBW; b++) {
+            if (b >= nbl) break;            // wave-uniform
+            const bool last = b + 1 >= nbl, refill = !last || xr;
+            const int nb = last ? 0 : b + 1;
+            if (last && xr) point(nxt);
+#pragma unroll
+            for (int r = 0; r < RG; r++) {
+                if (cur.p0 == cur.pb) wr[b][r].settle();
+                wr[b][r].hold();
+                floatx4 t = KRK_ZERO4;
+#define KRK_PAIR(P)                                                   \
+    __builtin_amdgcn_sched_barrier(0);                                \
+    wr[b][r].template pair<P>(xa[P], masks, t, acc[r]);               \
+    settle_acc(DT == DT_Q4_K || DT == DT_Q5_K ? t : acc[r]);          \
+    if (r == RG - 1 && refill) load_pair(P, nb);                      \
+    __builtin_amdgcn_sched_barrier(0);
+                KRK_PAIR(0) KRK_PAIR(1) KRK_PAIR(2) KRK_PAIR(3)
+#undef KRK_PAIR
+                wr[b][r].finish(xs, masks, t, acc[r]);
+                settle_acc(acc[r]);
+                if (r == RG - 1 && refill) load_sums(nb);
+                if (wn) fetch(nxt, b, r);
+            }
+        }
+        float *red = red_lds + buf * (nw * 16 * S);
+#pragma unroll
+        for (int r = 0; r < RG; r++)
+#pragma unroll
+            for (int k = 0; k < 4; k++) red[(wv * 16 + 4 * g + k) * S + 16 * r + j] = acc[r][k];
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        const int64_t n0 = static_cast<int64_t>(cur.tile) * rows_t;
+        for (int o = tid; o < left * rows_t; o += 64 * nw) {
+            const int i = o >> rows_sh, c = o - (i << rows_sh), p = cur.p0 + i;
+            const int64_t n = n0 + c;
+            if (o != tid) inv = a.inv[a.tok ? a.tok[p] : p];
+            if (n >= n_out) continue;
+            float v = wave_sums<NWMAX, NWX>(red + i * S + c, 16 * S, 8 * S, nw, a.planes) * inv;
+            if (pair) {
+                float up = wave_sums<NWMAX, NWX>(red + i * S + 16 * H + c, 16 * S, 8 * S, nw, a.planes) * inv;
+                if (a.act_f16) {
+                    // both dots rounded to f16 first, silu with the device
+                    // exponential (moe_table.hpp:250-253)
+                    v = static_cast<float>(static_cast<_Float16>(v));
+                    up = static_cast<float>(static_cast<_Float16>(up));
+                    v = silu_f(v) * up;
+                } else {
+                    v = (v / (1.0f + expf(-v))) * up;
+                }
+            }
+            out[p * n_out + n] = v;
+        }
+        if (end) break;
+        cur = nxt;
+    }
+}
+
+template <int DT, int RG> hipError_t launch(const RowsArgs &a, dim3 grid, int nw, hipStream_t st) {
     const size_t lds = static_cast<size_t>(nw) * 16 * (16 * RG + 4) * sizeof(float);
     if (nw == 8)
-        hipLaunchKernelGGL((rows_kernel<DT, NBW, RG, 8, true, DENSE>), grid, dim3(64 * nw), lds, st, a);
+        hipLaunchKernelGGL((rows_kernel<DT, RG, 8, true>), grid, dim3(64 * nw), lds, st, a);
     else if (nw < 8)
-        hipLaunchKernelGGL((rows_kernel<DT, NBW, RG, 8, false, DENSE>), grid, dim3(64 * nw), lds, st, a);
+        hipLaunchKernelGGL((rows_kernel<DT, RG, 8, false>), grid, dim3(64 * nw), lds, st, a);
     else if (nw == kRowsWaves)
-        hipLaunchKernelGGL((rows_kernel<DT, NBW, RG, kRowsWaves, true, DENSE>), grid, dim3(64 * nw), lds, st, a);
+        hipLaunchKernelGGL((rows_kernel<DT, RG, kRowsWaves, true>), grid, dim3(64 * nw), lds, st, a);
     else
-        hipLaunchKernelGGL((rows_kernel<DT, NBW, RG, kRowsWaves, false, DENSE>), grid, dim3(64 * nw), lds, st, a);
+        hipLaunchKernelGGL((rows_kernel<DT, RG, kRowsWaves, false>), grid, dim3(64 * nw), lds, st, a);
+    return hipGetLastError();
+}
+
+template <int DT, int NBW, int RG>
+hipError_t launch_routed(const RowsArgs &a, int nw, hipStream_t st) {
+    const size_t lds = static_cast<size_t>(2) * nw * 16 * (16 * RG + 4) * sizeof(float);
+    const int64_t rows_t = 16 * (a.pair ? RG / 2 : RG);
+    if (rows_t < 1 || a.max_runs < 1) return hipErrorNotSupported;
+    const int64_t tiles = (a.seg[0].n_out + rows_t - 1) / rows_t;
+    if (tiles * a.max_runs >= (int64_t{1} << 31)) return hipErrorNotSupported;
+    // as many workgroups as are resident (the registers allow sixteen waves a
+    // compute unit), chunks of up to eight tiles while every one gets four
+    const int64_t wgs = static_cast<int64_t>(device_cus()) * (nw <= 4 ? 4 : nw <= 5 ? 3 : nw <= 8 ? 2 : 1);
+    int64_t ct = tiles * a.max_runs / (4 * wgs);
+    ct = ct < 1 ? 1 : ct > 8 ? 8 : ct;
+    const int64_t chunks = (tiles + ct - 1) / ct * a.max_runs;
+    const dim3 grid(static_cast<unsigned>(chunks < wgs ? chunks : wgs));
+    const int t = static_cast<int>(tiles), c = static_cast<int>(ct);
+    if (nw == 8)
+        hipLaunchKernelGGL((rows_routed_kernel<DT, NBW, RG, 8, true>), grid, dim3(64 * nw), lds, st, a, t, c);
+    else if (nw < 8)
+        hipLaunchKernelGGL((rows_routed_kernel<DT, NBW, RG, 8, false>), grid, dim3(64 * nw), lds, st, a, t, c);
+    else if (nw == kRowsWaves)
+        hipLaunchKernelGGL((rows_routed_kernel<DT, NBW, RG, kRowsWaves, true>), grid, dim3(64 * nw), lds, st, a, t, c);
+    else
+        hipLaunchKernelGGL((rows_routed_kernel<DT, NBW, RG, kRowsWaves, false>), grid, dim3(64 * nw), lds, st, a, t, c);
     return hipGetLastError();
 }
 
@@ -725,10 +866,8 @@ RowsShape rows_shape(const RowsArgs &a, int dt, int nb) {   // (reads runs, n an
     // (Q6_K's and Q8_0's blocks of four row groups do not fit the registers)
     const bool wide = dt != DT_Q8_0 && dt != DT_Q6_K;
     if (a.runs) {
-        // a stream of workgroups: two of eight waves per compute unit, so one
-        // loads while the other multiplies
-        s.nbw = nb <= (dt == DT_Q8_0 ? 16 : 8) ? 1 : nb <= 16 ? 2 : (nb + kRowsWaves - 1) / kRowsWaves;
-        s.rg = s.nbw == 1 ? (wide ? 4 : 2) : nb <= 32 ? 2 : 1;
+        s.nbw = (nb + kRowsWaves - 1) / kRowsWaves;
+        s.rg = s.nbw == 1 ? (wide ? 4 : 2) : s.nbw == 2 ? 2 : 1;
         s.splits = 1;
         s.range = nb;
     } else {
@@ -746,26 +885,25 @@ RowsShape rows_shape(const RowsArgs &a, int dt, int nb) {   // (reads runs, n an
 }
 
 template <int DT> hipError_t launch_shape(const RowsArgs &a, const RowsShape &s, hipStream_t st) {
+    constexpr bool WIDE = DT != DT_Q8_0 && DT != DT_Q6_K;
+    if (a.runs) {
+        switch (s.nbw) {
+            case 1: return launch_routed<DT, 1, WIDE ? 4 : 2>(a, s.nw, st);
+            case 2: return launch_routed<DT, 2, 2>(a, s.nw, st);
+            case 3: return launch_routed<DT, 3, 1>(a, s.nw, st);
+            case 4: return launch_routed<DT, 4, 1>(a, s.nw, st);
+            default: return hipErrorNotSupported;
+        }
+    }
     int64_t widest = 0;
-    for (int i = 0; i < (a.runs ? 1 : a.n); i++) widest = a.seg[i].n_out > widest ? a.seg[i].n_out : widest;
-    const int64_t rows_t = 16 * (a.pair ? s.rg / 2 : s.rg);
-    if (rows_t < 1) return hipErrorNotSupported;
-    const int64_t width = (widest + rows_t - 1) / rows_t, ny = a.runs ? a.max_runs : a.n;
-    if (width >= (int64_t{1} << 31) || ny > 65535 || (s.splits > 1 && (!a.part || width * ny > kTileCounters)))
+    for (int i = 0; i < a.n; i++) widest = a.seg[i].n_out > widest ? a.seg[i].n_out : widest;
+    const int64_t width = (widest + 16 * s.rg - 1) / (16 * s.rg);
+    if (width >= (int64_t{1} << 31) || (s.splits > 1 && (!a.part || width * a.n > kTileCounters)))
         return hipErrorNotSupported;
-    const dim3 grid(static_cast<unsigned>(width), static_cast<unsigned>(ny), static_cast<unsigned>(s.splits));
-    if (!a.runs) {
-        if constexpr (DT != DT_Q8_0 && DT != DT_Q6_K)
-            if (s.rg == 4) return launch<DT, 1, 4, true>(a, grid, s.nw, st);
-        return s.rg == 2 ? launch<DT, 1, 2, true>(a, grid, s.nw, st) : launch<DT, 1, 1, true>(a, grid, s.nw, st);
-    }
-    switch (s.nbw) {
-        case 1: return launch<DT, 1, DT != DT_Q8_0 && DT != DT_Q6_K ? 4 : 2, false>(a, grid, s.nw, st);
-        case 2: return launch<DT, 2, 2, false>(a, grid, s.nw, st);
-        case 3: return launch<DT, 3, 1, false>(a, grid, s.nw, st);
-        case 4: return launch<DT, 4, 1, false>(a, grid, s.nw, st);
-        default: return hipErrorNotSupported;
-    }
+    const dim3 grid(static_cast<unsigned>(width), static_cast<unsigned>(a.n), static_cast<unsigned>(s.splits));
+    if constexpr (WIDE)
+        if (s.rg == 4) return launch<DT, 4>(a, grid, s.nw, st);
+    return s.rg == 2 ? launch<DT, 2>(a, grid, s.nw, st) : launch<DT, 1>(a, grid, s.nw, st);
 }
 
 }  // namespace
@@ -793,7 +931,7 @@ bool gemm_rows_ok(int dt, int64_t n_in, const void *w, int64_t row_bytes) {
             break;
         default: return false;
     }
-    return n_in > 0 && n_in % 256 == 0 && n_in / 256 <= kRowsWaves * kRowsBlocks;
+    return n_in > 0 && n_in % 256 == 0 && n_in / 256 <= kRowsWaves * kRowsBlocks;   // (rows well under 2^26 bytes)
 }
 
 static size_t prep_rows_bytes(int64_t rows, int64_t n_in, int planes, bool dense) {
