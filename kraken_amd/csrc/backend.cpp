@@ -414,7 +414,7 @@ int gemm_impl(krk_backend *b, void *out, const void *x, const void *w, int wt, i
     }
     // a fixed scratch needs the least the GEMM runs with; the growing
     // workspace takes what its fastest form needs
-    const size_t need = krk::gemm_mfma_workspace(wt, rows, n_out, n_in, fixed);
+    const size_t need = krk::gemm_mfma_workspace(wt, f16, rows, n_out, n_in, fixed);
     if (fixed && need > ws_bytes)
         return fail(b, KRK_ERR_NOMEM, "mfma gemm needs %zu bytes of split-K scratch; the fixed scratch holds %zu",
                     need, ws_bytes);

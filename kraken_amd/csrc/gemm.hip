@@ -123,6 +123,124 @@ struct Q4KPair {
     }
 };
 
+// Two codes as an f16 pair's bits (f16 subnormals q 2^-24, which the mixed
+// fma widens exactly) to weights f16(d q + c), d scaled by 2^24: one operation
+// a weight, rounded in f32 and then to f16 as the host decoder's value is.
+typedef _Float16 half2m __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void code_pair(uint32_t bits, float d24, float c, _Float16 &a, _Float16 &b) {
+    const half2m h = __builtin_bit_cast(half2m, bits);
+    a = static_cast<_Float16>(__builtin_fmaf(d24, static_cast<float>(h.x), c));
+    b = static_cast<_Float16>(__builtin_fmaf(d24, static_cast<float>(h.y), c));
+}
+// four byte codes to four weights
+__device__ __forceinline__ void code_bytes(uint32_t w, float d24, float c, _Float16 *o) {
+    code_pair(w & 0x00FF00FFu, d24, c, o[0], o[2]);
+    code_pair((w >> 8) & 0x00FF00FFu, d24, c, o[1], o[3]);
+}
+constexpr float kSub = 16777216.0f;   // 2^24
+
+// Q5_K by chunk pair, as Q4_K, with the 16 high-bit bytes of the slice's
+// positions (chunk c takes bit c of each as bit 4 of its code,
+// quant.cpp:462-489).  Three loads serve 32 weights, where each half-chunk
+// fetched its own header and high bits (six); 2048 f16 rows, 4096 -> 14336:
+// 354.7 -> 290.1 us.
+struct Q5KPair {
+    u32x4 hdr, q, hb;
+    __device__ void fetch(const uint8_t *row, int p, int h) {
+        const uint8_t *b = row + (p >> 2) * 176;
+        hdr = ld128(b);
+        hb = ld128(b + 16 + 16 * h);
+        q = ld128(b + 48 + 32 * (p & 3) + 16 * h);
+    }
+    __device__ void decode(int p, _Float16 (&lo)[16], _Float16 (&hi)[16]) const {
+        const float d = h2f(hdr.x & 0xFFFF), dmin = h2f(hdr.x >> 16);
+        const uint32_t h4[4] = {hdr.x, hdr.y, hdr.z, hdr.w};
+        uint32_t sa, sb, ma, mb;
+        q4k_pair_scale_bytes(h4, p & 3, sa, sb, ma, mb);
+        const float d1a = kSub * (d * static_cast<float>(sa)), m1a = dmin * static_cast<float>(ma);
+        const float d1b = kSub * (d * static_cast<float>(sb)), m1b = dmin * static_cast<float>(mb);
+        const int c = 2 * (p & 3);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            // the high bits of both chunks at bits 4 and 5 of each byte
+            const uint32_t two = (hb[t] >> c) << 4;
+            code_bytes((q[t] & 0x0F0F0F0Fu) | (two & 0x10101010u), d1a, -m1a, &lo[4 * t]);
+            code_bytes(((q[t] >> 4) & 0x0F0F0F0Fu) | ((two >> 1) & 0x10101010u), d1b, -m1b, &hi[4 * t]);
+        }
+    }
+};
+
+// Q6_K by chunk pair: step p is quadrants 2 (p % 2) and 2 (p % 2) + 1 of half
+// (p / 2) % 2 of block p / 4.  The thread with slice h takes positions
+// 16 h .. + 15 of both: their ql bytes (one nibble of each) and the qh bytes
+// they share: five loads (unaligned 16-byte ones) for 32 weights, where the
+// half-chunks' dword windows took 24; 2048 f16 rows, 4096 -> 14336: 596.9 ->
+// 463.1 us (what is left over Q4_K's 274 is the unaligned loads).
+struct Q6KPair {
+    u32x4 la, lb, hb;
+    uint32_t sw, dw;
+    __device__ void fetch(const uint8_t *row, int p, int h) {
+        const int hh = (p >> 1) & 1, pr = p & 1;
+        gbyte *b = to_global(row + (p >> 2) * 210);
+        la = ld128_a2(b + 64 * hh + 16 * h);
+        lb = ld128_a2(b + 64 * hh + 32 + 16 * h);
+        hb = ld128_a2(b + 128 + 32 * hh + 16 * h);
+        // scales 8 hh + 4 pr + h and + 2 (the 4 bytes end at 203 at most)
+        sw = ld32_a2(b + 192 + 8 * hh + 4 * pr) >> (8 * h);
+        dw = ld16g(b + 208);
+    }
+    __device__ void decode(int p, _Float16 (&lo)[16], _Float16 (&hi)[16]) const {
+        const int pr = p & 1;
+        const float d = h2f(dw);
+        const float da = d * static_cast<float>(static_cast<int8_t>(sw & 0xFF));
+        const float db = d * static_cast<float>(static_cast<int8_t>((sw >> 16) & 0xFF));
+        const float a24 = kSub * da, b24 = kSub * db, ca = -32.0f * da, cb = -32.0f * db;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const uint32_t h = hb[t] >> (4 * pr);   // bits 0..1: the even quadrant, 2..3: the odd one
+            code_bytes(((la[t] >> (4 * pr)) & 0x0F0F0F0Fu) | ((h << 4) & 0x30303030u), a24, ca, &lo[4 * t]);
+            code_bytes(((lb[t] >> (4 * pr)) & 0x0F0F0F0Fu) | ((h << 2) & 0x30303030u), b24, cb, &hi[4 * t]);
+        }
+    }
+};
+
+// Q8_0 and Q4_0: a thread's 32-value chunk is one block
+struct Q8Chunk {
+    u32x4 q0, q1;
+    uint32_t dw;
+    __device__ void fetch(const uint8_t *row, int c) {
+        gbyte *b = to_global(row + c * 34);
+        dw = ld16g(b);
+        q0 = ld128_a2(b + 2);
+        q1 = ld128_a2(b + 18);
+    }
+    __device__ void decode(_Float16 (&lo)[16], _Float16 (&hi)[16]) const {
+        const float d24 = kSub * h2f(dw), c = -128.0f * h2f(dw);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            code_bytes(q0[t] ^ 0x80808080u, d24, c, &lo[4 * t]);
+            code_bytes(q1[t] ^ 0x80808080u, d24, c, &hi[4 * t]);
+        }
+    }
+};
+struct Q40Chunk {
+    u32x4 q;
+    uint32_t dw;
+    __device__ void fetch(const uint8_t *row, int c) {
+        gbyte *b = to_global(row + c * 18);
+        dw = ld16g(b);
+        q = ld128_a2(b + 2);
+    }
+    __device__ void decode(_Float16 (&lo)[16], _Float16 (&hi)[16]) const {
+        const float d24 = kSub * h2f(dw), c = -8.0f * h2f(dw);
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            code_bytes(q[t] & 0x0F0F0F0Fu, d24, c, &lo[4 * t]);
+            code_bytes((q[t] >> 4) & 0x0F0F0F0Fu, d24, c, &hi[4 * t]);
+        }
+    }
+};
+
 template <> struct WStage<DT_Q6_K> {
     uint32_t ql[4], qh[4], sw, dw;
     __device__ void fetch(const uint8_t *row, int kt, int hf) {
@@ -487,6 +605,26 @@ template <typename XT> struct StepRegs<DT_Q4_K, XT> {
     Q4KPair w;
     XStage<XT> x0, x1;
 };
+template <typename XT> struct StepRegs<DT_Q5_K, XT> {
+    Q5KPair w;
+    XStage<XT> x0, x1;
+};
+template <typename XT> struct StepRegs<DT_Q6_K, XT> {
+    Q6KPair w;
+    XStage<XT> x0, x1;
+};
+template <typename XT> struct StepRegs<DT_Q8_0, XT> {
+    Q8Chunk w;
+    XStage<XT> x0, x1;
+};
+template <typename XT> struct StepRegs<DT_Q4_0, XT> {
+    Q40Chunk w;
+    XStage<XT> x0, x1;
+};
+// formats staged by chunk pair (a thread: one slice of both chunks), and by
+// whole chunk
+constexpr bool by_pair(int dt) { return dt == DT_Q4_K || dt == DT_Q5_K || dt == DT_Q6_K; }
+constexpr bool by_chunk(int dt) { return dt == DT_Q8_0 || dt == DT_Q4_0; }
 
 // Whether a (format, activation type) pair keeps two steps of raw bytes in
 // registers without spilling (256 VGPRs at two waves per SIMD; measured on
@@ -539,9 +677,11 @@ __global__ void __launch_bounds__(G_THREADS, 1)
         const int c = c0 + 2 * it;
         const bool ok = c < cend;
         const int cc = ok ? c : cend - 1;          // stay inside the row
-        if constexpr (DT == DT_Q4_K) {
+        if constexpr (by_pair(DT)) {
             const int pp = c >> 1;                  // chunk pair of this step
             r.w.fetch(wrow, 2 * pp < cend ? pp : (cend - 1) >> 1, shf);
+        } else if constexpr (by_chunk(DT)) {
+            r.w.fetch(wrow, cc);
         } else {
             r.w0.fetch(wrow, cc, 0);
             r.w1.fetch(wrow, cc, 1);
@@ -554,9 +694,9 @@ __global__ void __launch_bounds__(G_THREADS, 1)
         const int c = c0 + 2 * it;
         _Float16 a[16], b[16];
         // a, b: the two 16-value runs this thread stores, at wo and wo + 16
-        // (Q4_K: slice shf of the even chunk at 16 shf, of the odd at 32 + 16 shf)
+        // (pairs: slice shf of the even chunk at 16 shf, of the odd at 32 + 16 shf)
         int wo = shf * 32, bo = shf * 32 + 16;
-        if constexpr (DT == DT_Q4_K) {
+        if constexpr (by_pair(DT)) {
             const int pp = c >> 1;
             r.w.decode(pp, a, b);
             if (2 * pp + 1 >= cend) {   // the half step past K: zero the odd chunk
@@ -566,8 +706,12 @@ __global__ void __launch_bounds__(G_THREADS, 1)
             wo = 16 * shf;
             bo = 32 + 16 * shf;
         } else {
-            r.w0.decode(c, a);
-            r.w1.decode(c, b);
+            if constexpr (by_chunk(DT)) {
+                r.w.decode(a, b);
+            } else {
+                r.w0.decode(c, a);
+                r.w1.decode(c, b);
+            }
             if (c >= cend) {   // the half step past K: zero weights (the activations are zero too)
 #pragma unroll
                 for (int i = 0; i < 16; i++) { a[i] = static_cast<_Float16>(0.0f); b[i] = a[i]; }
@@ -835,7 +979,17 @@ static size_t splitk_floats(int64_t M, int64_t N, int s, bool images) {
     return tiles * s * GB_M * GB_N;
 }
 
-size_t gemm_mfma_workspace(int dt, int64_t M, int64_t N, int64_t K, bool minimal) {
+// f32 rows as f16 before the tile GEMM (each N tile would convert them again,
+// and read twice the bytes; the shorter staging registers also let every
+// format prefetch two steps): formats that are worth a third kernel.
+// Measured, 2048 f32 rows, 4096 -> 14336: Q4_K 423.7 -> 288.9 us, Q5_K 520.5
+// -> 302.2, Q6_K 771.9 -> 472.8, Q8_0 650.7 -> 457.5, Q4_0 615.9 -> 392.9
+// (Q5_K and Q6_K with their pair stagings)
+static bool rows_once(int dt) {
+    return dt == DT_Q4_K || dt == DT_Q5_K || dt == DT_Q6_K || dt == DT_Q8_0 || dt == DT_Q4_0;
+}
+
+size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal) {
     if (stream_gemm(dt, M, N, K)) {   // f32 rows as f16, and the split partials
         const int s = stream_split(M, N, K);
         return al256(static_cast<size_t>(M * K) * sizeof(_Float16)) +
@@ -843,7 +997,8 @@ size_t gemm_mfma_workspace(int dt, int64_t M, int64_t N, int64_t K, bool minimal
     }
     const int s = pick_split(M, N, K, dt);
     const size_t flat = splitk_floats(M, N, s, false), imgs = splitk_floats(M, N, s, true);
-    return (minimal || flat > imgs ? flat : imgs) * sizeof(float);
+    const size_t part = (minimal || flat > imgs ? flat : imgs) * sizeof(float);
+    return minimal || act_f16 || !rows_once(dt) ? part : al256(part) + static_cast<size_t>(M * K) * sizeof(_Float16);
 }
 
 template <int DT, typename XT, typename OT>
@@ -882,7 +1037,7 @@ hipError_t gemm_mfma(int dt, const void *w, int64_t row_bytes, const void *x, bo
                      void *out, int64_t M, int64_t N, int64_t K, void *ws, size_t ws_bytes,
                      unsigned *cnt, hipStream_t st) {
     if (stream_gemm(dt, M, N, K)) {
-        if (ws_bytes < gemm_mfma_workspace(dt, M, N, K, false)) return hipErrorInvalidValue;
+        if (ws_bytes < gemm_mfma_workspace(dt, act_f16, M, N, K, false)) return hipErrorInvalidValue;
         const int split = stream_split(M, N, K);
         float *part = reinterpret_cast<float *>(static_cast<uint8_t *>(ws) +
                                                 al256(static_cast<size_t>(M * K) * sizeof(_Float16)));
@@ -913,6 +1068,29 @@ hipError_t gemm_mfma(int dt, const void *w, int64_t row_bytes, const void *x, bo
             hipLaunchKernelGGL((splitk_reduce_kernel<float>), dim3(static_cast<unsigned>((MN + 2047) / 2048)),
                                dim3(256), 0, st, part, static_cast<float *>(out), MN, split);
         return hipGetLastError();
+    }
+    if (!act_f16 && rows_once(dt)) {
+        const size_t xb = static_cast<size_t>(M * K) * sizeof(_Float16);
+        // the rows go behind the split-K scratch; a fixed scratch that does not
+        // hold them keeps the f32 staging
+        const size_t need = gemm_mfma_workspace(dt, false, M, N, K, true);
+        if (ws_bytes >= al256(need) + xb) {
+            const size_t at = (ws_bytes - xb) & ~size_t(255);
+            _Float16 *xh = reinterpret_cast<_Float16 *>(static_cast<uint8_t *>(ws) + at);
+            const hipError_t e = moe_gather_f16(static_cast<const float *>(x), K, nullptr, nullptr, M, xh, st);
+            if (e != hipSuccess) return e;
+            switch (dt) {
+#define KRK_GEMM_ONCE(D) \
+    case D: return launch_f16<D, _Float16, float>(w, row_bytes, xh, out, M, N, K, ws, at, cnt, st);
+                KRK_GEMM_ONCE(DT_Q4_K)
+                KRK_GEMM_ONCE(DT_Q5_K)
+                KRK_GEMM_ONCE(DT_Q6_K)
+                KRK_GEMM_ONCE(DT_Q8_0)
+                KRK_GEMM_ONCE(DT_Q4_0)
+#undef KRK_GEMM_ONCE
+                default: return hipErrorInvalidValue;
+            }
+        }
     }
 #define KRK_GEMM_CASE(D)                                                                       \
     case D:                                                                                   \

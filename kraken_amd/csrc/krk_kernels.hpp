@@ -155,7 +155,7 @@ hipError_t quantize_q8_rows_f16codes(const void *x, bool x_f16, int64_t rows, in
 // out[M, N] = X[M, K] . deq(W)[N, K]^T.  `ws` is device scratch of ws_bytes.
 // scratch of gemm_mfma: what its fastest form needs, or (minimal) the
 // least it runs with
-size_t gemm_mfma_workspace(int dt, int64_t M, int64_t N, int64_t K, bool minimal);
+size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal);
 // compute units of the current device (cached on first use)
 int device_cus();
 // cnt: kTileCounters zeroed counters owned by the caller (left zero after

@@ -173,3 +173,24 @@ def test_rows_moe_f16(krk, torch_cuda, be16, dt, n_tok, n_embd, n_ff):
     assert rel(got.astype(np.float32), ref.astype(np.float32)) <= 3e-4
     assert (f16_ulps(got, ref) == 0).mean() >= 0.8
     be16.moe_table_forget(table)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+def test_tile_gemm_f32_rows(krk, torch_cuda, be32, dt):
+    """The tile GEMM's f32 rows, rounded to f16 before it (krk_gemm) or while
+    staged (a fixed scratch that does not hold them): the same f16 operands in
+    the same order, so bit-equal, and within the MFMA bar of the oracle."""
+    torch = torch_cuda
+    rows, n_out, n_in = 2050, 260, 16384     # 2050 x 16384 f16 rows: 64.1 MiB
+    assert rows * n_in * 2 > krk.lib().krk_gemm_noalloc_scratch_bytes()
+    w = make_weights(krk, dt, n_out, n_in, seed=9)
+    x = krk.synth_normal(rows * n_in, seed=10).reshape(rows, n_in)
+    xd, wd = dev(torch, x), dev(torch, w)
+    a = torch.full((rows, n_out), float("nan"), dtype=torch.float32, device="cuda")
+    b = torch.full_like(a, float("nan"))
+    be32.gemm(a, xd, wd, dt, n_out, n_in, rows)
+    be32.gemm_noalloc(b, xd, wd, dt, n_out, n_in, rows)
+    be32.sync()
+    assert torch.equal(a, b)
+    pick = [0, 1, 255, 256, 1000, 2049]
+    assert rel(host(a)[pick], O.gemm(dt, w, x[pick], n_out, nthreads=16)) <= GEMM_TOL
