@@ -92,15 +92,29 @@ static MoeWs carve(void *ws, int64_t P, int ne, int64_t n_embd, int64_t n_ff) {
     return w;
 }
 
+// f32 batches from this many tokens take the grouped expert GEMM when the
+// gemm path allows f16 products
+constexpr int64_t kMoeGemmTokens = 32;
+static bool moe_grouped(const MoeArgs &a) {
+    return a.mfma && !a.act_f16 && a.n_tok >= kMoeGemmTokens && a.aligned16 && a.wt >= 0 && a.rb_gate == a.rb_up &&
+           moe_gemm_ok(a.wt) && moe_gemm_ok(a.wt_down) && a.n_tok * a.k <= (1 << 24);
+}
+
 // Calls whose experts run on the rows kernel (gemm_rows.hip): exact products
 // over each active expert's tokens, its banks streamed once.  Layers of one
-// gate/up type and one down type among Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0;
-// kRowsMoeF32: the f32 batches it takes (below, with the figures).
+// gate/up type and one down type among Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0, with
+// f16 activations, and with f32 ones where the grouped GEMM does not apply.
+// f32 Q4_K gate/up layers keep the streaming GEMV's runs (one token at a time)
+// below 7 pairs in 4 experts.  Measured at 128 experts, 4096 / 1536, top 8
+// (us, rows kernel against the path before): f32 Q8_0 1 token 90 (148), 16
+// tokens 599 (1234), Q5_K / Q6_K 16 tokens 384 (1529), Q4_K 16 tokens 250
+// (247), 31 tokens 311 (350), 512 tokens under KRK_PATH_EXACT 1338 (2441).
 static bool moe_rows(const MoeArgs &a) {
-    if (a.wt < 0 || a.rb_gate != a.rb_up || !a.aligned16 || a.n_embd > 8192) return false;
+    if (a.wt < 0 || a.rb_gate != a.rb_up || !a.aligned16 || a.n_embd > 8192 || moe_grouped(a)) return false;
     if (!gemm_rows_ok(a.wt, a.n_embd, nullptr, a.rb_gate) || !gemm_rows_ok(a.wt_down, a.n_ff, nullptr, a.rb_down))
         return false;
-    return a.act_f16;
+    const bool runs = a.wt == DT_Q4_K && (a.wt_down == DT_Q4_K || a.wt_down == DT_Q6_K) && a.k <= kMaxSegs;
+    return a.act_f16 || !runs || 4 * a.n_tok * a.k >= 7 * a.n_expert;
 }
 
 size_t moe_workspace(const MoeArgs &a) {
@@ -550,9 +564,6 @@ __global__ void __launch_bounds__(512) moe_down1_kernel(const krk_moe_entry *__r
 }
 
 constexpr int64_t kMoeTokenGroups = 64;
-// f32 batches from this many tokens take the grouped expert GEMM when the
-// gemm path allows f16 products
-constexpr int64_t kMoeGemmTokens = 32;
 
 hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t st) {
     const int64_t P = a.n_tok * a.k;
@@ -643,8 +654,7 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
     // mi (1 or 2) from the mean pairs per active expert, then the ordered
     // reduce.
     // f16 operands and f32 accumulation, as the dense GEMM above 8 rows.
-    if (a.mfma && !a.act_f16 && a.n_tok >= kMoeGemmTokens && a.aligned16 && a.wt >= 0 &&
-        a.rb_gate == a.rb_up && moe_gemm_ok(a.wt) && moe_gemm_ok(a.wt_down) && P <= (1 << 24)) {
+    if (moe_grouped(a)) {
         const int64_t act = P < a.n_expert ? P : a.n_expert;
         const int64_t per = (P + act - 1) / act;
         const int mi = per <= 21 ? 1 : 2;

@@ -194,3 +194,31 @@ def test_tile_gemm_f32_rows(krk, torch_cuda, be32, dt):
     assert torch.equal(a, b)
     pick = [0, 1, 255, 256, 1000, 2049]
     assert rel(host(a)[pick], O.gemm(dt, w, x[pick], n_out, nthreads=16)) <= GEMM_TOL
+
+
+@pytest.mark.parametrize("dt", [O.Q8_0, (O.Q5_K, O.Q5_K, O.Q6_K), O.Q4_0, O.Q4_K])
+@pytest.mark.parametrize("n_tok", [1, 5, 40])
+def test_rows_moe_f32(krk, torch_cuda, be32, dt, n_tok):
+    """f32 rows as two planes, one and several passes of eight rows (40 tokens
+    under KRK_PATH_EXACT), dropped slots: the GEMV bar."""
+    torch = torch_cuda
+    ne, n_embd, n_ff, k = 6, 768, 1024, 3
+    mats, table, keep = build_moe(krk, torch, dt, ne, n_embd, n_ff, seed=1950)
+    ids, wts = O.router_topk(O.router_softmax(krk.synth_normal(n_tok * ne, seed=187).reshape(n_tok, ne)), k)
+    if n_tok > 1:
+        ids[0, 1] = -1
+    x = krk.synth_normal(n_tok * n_embd, seed=188).reshape(n_tok, n_embd)
+    x[n_tok // 2] *= 1e4
+    say("rows moe f32", dt, n_tok)
+    out = torch.full((n_tok, n_embd), float("nan"), dtype=torch.float32, device="cuda")
+    be32.set_gemm_path(krk.PATH_EXACT)
+    try:
+        be32.moe_dispatch(table, 0, ne, dev(torch, ids), dev(torch, wts), dev(torch, x), out, n_tok, n_embd, n_ff, k)
+        be32.sync()
+    finally:
+        be32.set_gemm_path(krk.PATH_AUTO)
+        be32.moe_table_forget(table)
+    ref = O.moe_ffn(x, [mats[0, e] for e in range(ne)], [mats[1, e] for e in range(ne)],
+                    [mats[2, e] for e in range(ne)], dt, ids, wts, n_ff)
+    for t in range(n_tok):
+        assert rel(host(out)[t], ref[t]) <= GEMV_TOL, t
