@@ -174,12 +174,15 @@ __global__ void __launch_bounds__(64) stream_xtab_kernel(const XT *__restrict__ 
 // activation rows concatenated; a wave's slice lies in one slot, whose bank
 // it reads and whose routing weight scales its activations); 3 and 4
 // expert-major runs (gate/up pairs, down): grid row a = active expert
-// em_runs[a], its weights loaded once and applied to each of its rows in turn
+// em_runs[a], its weights loaded once and applied to each of its rows in turn;
+// 5 the routed down projection of one token slot by slot (f16 activations,
+// whose partial results are rounded per slot before they are added): grid row
+// s = slot s, its activations row s, its f32 outputs row s
 template <int DT, typename XT, typename OT, int NBW, int TR, int NWMAX, bool NWEXACT, int MOE = 0, int LA = 8,
           int XR = 1, bool LT = false>
 // (the second bound is waves per SIMD: four for the expert-major runs and
 // for five rows, whose registers would otherwise leave one workgroup per CU)
-__global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8) ? 4 : 1)
+__global__ void __launch_bounds__(64 * NWMAX, MOE == 3 || MOE == 4 || (XR > 4 && NWMAX == 8) ? 4 : 1)
     gemv_stream_kernel(SegTable t) {
     // XR: activation rows (dense Q4_K launches of 2..5 rows): every row's
     // activations load before the weights, one digit table per row, each
@@ -187,9 +190,10 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
     static_assert(XR == 1 || (MOE == 0 && DT == DT_Q4_K), "several rows: dense Q4_K");
     // LT: the weights move as lane-contiguous 16-byte pieces (full cache
     // lines, nontemporal) and are transposed through the wave's LDS
-    static_assert(!LT || ((DT == DT_Q4_K || DT == DT_Q6_K || DT == DT_Q4_0 || DT == DT_Q8_0) && MOE < 3),
+    static_assert(!LT || ((DT == DT_Q4_K || DT == DT_Q6_K || DT == DT_Q4_0 || DT == DT_Q8_0) && MOE != 3 && MOE != 4),
                   "load-transpose: Q4_K, Q6_K, Q4_0 or Q8_0, dense or routed");
     using LTG = LtGeom<NBW, TR, DT == DT_Q6_K ? 14 : DT == DT_Q8_0 ? 17 : 9>;
+    constexpr bool EM = MOE == 3 || MOE == 4;
     constexpr bool Q6 = DT == DT_Q6_K;
     constexpr bool Q40 = DT == DT_Q4_0;
     constexpr bool Q80 = DT == DT_Q8_0;
@@ -238,6 +242,12 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
         w = static_cast<const uint8_t *>(en.p[KRK_MOE_GATE]);
         w2s = static_cast<const uint8_t *>(en.p[KRK_MOE_UP]);
         outp += static_cast<int64_t>(blockIdx.y) * n_out;
+    } else if constexpr (MOE == 5) {
+        const int e = t.moe_ids[blockIdx.y];
+        const bool live = e >= 0 && e < t.moe_ne;
+        w = static_cast<const uint8_t *>(static_cast<const krk_moe_entry *>(t.moe_tab)[live ? e : 0].p[KRK_MOE_DOWN]);
+        x += static_cast<int64_t>(blockIdx.y) * t.n_in;
+        outp += static_cast<int64_t>(blockIdx.y) * n_out;
     } else if constexpr (MOE == 2) {
         const int bps = static_cast<int>(t.moe_kslot >> 8);   // blocks per slot
         const int sl = kb0 / bps < t.moe_k ? kb0 / bps : t.moe_k - 1;
@@ -248,7 +258,7 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
         kblk = kb0 - sl * bps;
     }
     int pb = 0, pe = 1;   // the rows served: expert-major runs' plan positions
-    if constexpr (MOE >= 3) {
+    if constexpr (EM) {
         // the run record and the active count in one round of scalar loads
         const EmRun &run = t.em_runs[blockIdx.y];
         const int nact = *t.em_n_act;
@@ -259,7 +269,7 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
         if (static_cast<int>(blockIdx.y) >= nact) return;   // beyond the active experts
     }
     auto row_x = [&](int p) {
-        return MOE >= 3 ? x + static_cast<int64_t>(t.em_tok ? t.em_tok[p] : p) * t.em_xrow : x;
+        return EM ? x + static_cast<int64_t>(t.em_tok ? t.em_tok[p] : p) * t.em_xrow : x;
     };
     const uint8_t *w2 = pair ? w2s : w;
 
@@ -419,7 +429,7 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
 
     for (int pr = pb; pr < pe; pr++) {
     // (expert-major runs: every wave has read the previous row's sums)
-    if (MOE >= 3 && pr > pb) __syncthreads();
+    if (EM && pr > pb) __syncthreads();
     // ---- the digit table of the slice (this wave's own LDS), layout
     // [block][sub-block][plane][32 bytes], {2^-e, sum x} per sub-block, and
     // for Q6_K the exact integer sums of X over each 16-value half (int bits)
@@ -558,12 +568,12 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
 
     // (expert-major runs: the next row's activations load while this one
     // is multiplied)
-    if (MOE >= 3 && pr + 1 < pe) load_xrow(row_x(pr + 1));
+    if (EM && pr + 1 < pe) load_xrow(row_x(pr + 1));
     // two-block slices read their A operands once, before the first group
     // lands (wider slices read them per group: registers)
     // (expert-major runs keep their weights live across rows, several
     // activation rows need the registers too)
-    constexpr bool HOLD = NBW == 2 && !Q6 && MOE < 3 && XR == 1;
+    constexpr bool HOLD = NBW == 2 && !Q6 && !EM && XR == 1;
     v4i HA[HOLD ? NBW : 1][4];
     float2 HE[HOLD ? NBW : 1][2];
     if constexpr (HOLD) {
@@ -923,7 +933,7 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
             if (k < nw) v += red[rr * nw + k];
         return v;
     };
-    OT *o = outp + (MOE >= 3 ? static_cast<int64_t>(pr) * t.em_orow : 0) + xr * t.out_stride + n0 + r;
+    OT *o = outp + (EM ? static_cast<int64_t>(pr) * t.em_orow : 0) + xr * t.out_stride + n0 + r;
     if (kind == SEG_SILU) {
         const float gs = row_sum(r), us = row_sum(16 + r);
         if constexpr (sizeof(OT) == 2) {
@@ -932,6 +942,12 @@ __global__ void __launch_bounds__(64 * NWMAX, MOE >= 3 || (XR > 4 && NWMAX == 8)
             const float hg = static_cast<float>(static_cast<_Float16>(gs));
             const float hu = static_cast<float>(static_cast<_Float16>(us));
             *o = sat_f16(silu_f(hg) * hu);
+        } else if constexpr (sizeof(XT) == 2) {
+            // the f16 expert layer: both dots rounded to f16, the row kept in
+            // f32 for its scale (moe_table.hpp:250-253)
+            const float hg = static_cast<float>(static_cast<_Float16>(gs));
+            const float hu = static_cast<float>(static_cast<_Float16>(us));
+            *o = silu_f(hg) * hu;
         } else {
             *o = (gs / (1.0f + expf(-gs))) * us;   // silu_mul, backend_cpu.cpp:2401-2406
         }
@@ -969,14 +985,14 @@ hipError_t launch(const SegTable &t, int64_t tiles, int nw, hipStream_t st) {
     // (Q4_0: its 256-value groups are 144 bytes like Q4_K's blocks; Q8_0's
     // 272-byte groups fit the LDS up to eight waves (K <= 4096), and sixteen
     // waves keep register loads)
-    constexpr bool LT = XR == 1 && MOE < 3 &&
+    constexpr bool LT = XR == 1 && MOE != 3 && MOE != 4 &&
                         ((DT == DT_Q4_K && (NBW == 2 || (NBW == 3 && TR == 16))) ||
                          ((DT == DT_Q6_K || DT == DT_Q4_0 || DT == DT_Q8_0) && NBW == 2));
     constexpr bool LTW = LT && DT != DT_Q8_0;   // (over eight waves)
     const size_t l = stream_lds(nw, NBW, XR) +
                      ((nw <= 8 ? LT : LTW) ? stream_lt_lds(nw, NBW, TR, DT == DT_Q6_K ? 14 : DT == DT_Q8_0 ? 17 : 9) : 0);
     const dim3 grid(static_cast<unsigned>(tiles),
-                    static_cast<unsigned>(MOE == 2 ? 1 : MOE >= 3 ? t.em_max_items : t.n));
+                    static_cast<unsigned>(MOE == 2 ? 1 : MOE == 3 || MOE == 4 ? t.em_max_items : MOE == 5 ? t.moe_k : t.n));
     if (nw == 8)
         hipLaunchKernelGGL((gemv_stream_kernel<DT, XT, OT, NBW, TR, 8, true, MOE, 8, XR, LT>), grid, dim3(64 * nw), l, st,
                            t);
@@ -1042,7 +1058,7 @@ bool gemv_stream_ok(int dt, const SegTable &t) {
     if (t.moe_tab) {
         // Q4_K banks; the down bank may also be Q6_K (Q4_K_M layers: its
         // 210-byte blocks need only 2-byte aligned rows)
-        const bool down = t.moe_down || (t.em_runs && t.seg[0].kind == SEG_PLAIN);
+        const bool down = t.moe_down || t.moe_slots || (t.em_runs && t.seg[0].kind == SEG_PLAIN);
         if (!(dt == DT_Q4_K || (dt == DT_Q6_K && down)) || t.n_in % 256 || t.row_bytes % (dt == DT_Q6_K ? 2 : 16))
             return false;
         const int nb = t.n_in / 256, nbw = stream_nbw(nb);
@@ -1058,6 +1074,9 @@ bool gemv_stream_ok(int dt, const SegTable &t) {
         // blocks) or the down projection over the concatenated slots, each
         // wave's slice inside one slot
         if (t.moe_tokens > 1) return false;
+        if (t.moe_slots)
+            return t.n == 1 && t.moe_k >= 1 && t.moe_k <= 65535 && nb <= 4 * kMaxWaves && t.seg[0].kind == SEG_PLAIN &&
+                   (reinterpret_cast<uintptr_t>(t.seg[0].x) & 15) == 0;
         if (t.moe_down)
             return t.n == 1 && t.moe_k >= 1 && t.moe_kslot % 256 == 0 && t.n_in == t.moe_k * t.moe_kslot &&
                    (t.moe_kslot / 256) % nbw == 0 && nb <= 4 * kMaxWaves && t.seg[0].kind == SEG_PLAIN &&
@@ -1123,7 +1142,29 @@ hipError_t gemv_stream(int dt, bool act_f16, const SegTable &t0, hipStream_t st)
         // routed experts (f32 activations, Q4_K): gate/up pairs take 32-row
         // tiles (16 + 16), the down projection 16-row tiles when its slices
         // are wider than two blocks
-        if (act_f16 || !(dt == DT_Q4_K || dt == DT_Q6_K)) return hipErrorNotSupported;
+        if (!(dt == DT_Q4_K || dt == DT_Q6_K)) return hipErrorNotSupported;
+        if (act_f16) {
+            // one token with f16 activations: gate/up pairs into f32 rows, then
+            // the down projection slot by slot (16-row tiles: there are k
+            // times as many as the matrix alone has)
+            if (t.em_runs || t.moe_down) return hipErrorNotSupported;
+            const int64_t width = (t.seg[0].n_out + 15) / 16;
+            if (!t.moe_slots)
+                return dt == DT_Q4_K ? launch<DT_Q4_K, _Float16, float, 2, 32, 1>(t, width, nw, st) : hipErrorNotSupported;
+            if (dt == DT_Q4_K) {
+                switch (nbw) {
+                    case 2: return launch<DT_Q4_K, _Float16, float, 2, 16, 5>(t, width, nw, st);
+                    case 3: return launch<DT_Q4_K, _Float16, float, 3, 16, 5>(t, width, nw, st);
+                    default: return launch<DT_Q4_K, _Float16, float, 4, 16, 5>(t, width, nw, st);
+                }
+            }
+            switch (nbw) {
+                case 2: return launch<DT_Q6_K, _Float16, float, 2, 16, 5>(t, width, nw, st);
+                case 3: return launch<DT_Q6_K, _Float16, float, 3, 16, 5>(t, width, nw, st);
+                default: return launch<DT_Q6_K, _Float16, float, 4, 16, 5>(t, width, nw, st);
+            }
+        }
+        if (t.moe_slots) return hipErrorNotSupported;
         if (dt == DT_Q6_K) {   // the down bank of a Q4_K_M layer
             if (t.em_runs) {
                 if (t.seg[0].kind == SEG_SILU) return hipErrorNotSupported;

@@ -56,6 +56,10 @@ struct SegTable {
     int moe_down;
     int moe_k;
     int64_t moe_kslot;
+    // Slot mode (moe_slots, with moe_tab and one plain segment): grid row s is
+    // slot s of one token, its weights the down bank of expert moe_ids[s], its
+    // activations seg[0].x + s n_in, its f32 outputs seg[0].out + s n_out.
+    int moe_slots;
     // Several tokens (moe_tokens > 1): the grid is moe_tokens groups of
     // moe_wpt workgroups; group tk handles token tk: its ids and weights at
     // moe_ids / moe_wts + tk * k, its activations at seg[0].x + tk * moe_xtok

@@ -376,11 +376,12 @@ __global__ void __launch_bounds__(512) moe_down_kernel(const krk_moe_entry *__re
 // the down dot reads (moe_table_scale_kernel, moe_table.hpp:256-305): the
 // smallest scale >= 1 (at most 2^24) with max |mid| <= 65504 * scale, and
 // midf = f16(mid * (1 / scale)), the reciprocal exact.  One workgroup per
-// plan position; positions past the live pairs leave at once.
-__global__ void __launch_bounds__(256) moe_scale_kernel(int64_t n_ff, int ne, MoeWs w) {
+// plan position; positions past the live pairs leave at once.  (PLAN false:
+// one token, its slots' rows in slot order.)
+template <bool PLAN> __global__ void __launch_bounds__(256) moe_scale_kernel(int64_t n_ff, int ne, MoeWs w) {
     __shared__ float red[4];
     const int64_t p = blockIdx.x;
-    if (p >= w.off[ne]) return;
+    if (PLAN && p >= w.off[ne]) return;
     const float *row = w.mid + p * n_ff;
     float mx = 0.0f;
     for (int64_t j = threadIdx.x; j < n_ff; j += blockDim.x) mx = fmaxf(mx, fabsf(row[j]));
@@ -400,8 +401,11 @@ __global__ void __launch_bounds__(256) moe_scale_kernel(int64_t n_ff, int ne, Mo
 // (moe_table_reduce_kernel, moe_table.hpp:536-551, with the partial of
 // table_down_batch, 418-441): per slot s in order, part = w * (f16(v) *
 // scale), two round-to-nearest products, and a = f16(a + part); a dropped
-// slot adds nothing (a is already an f16 value).
-__global__ void __launch_bounds__(256) moe_reduce_f16_kernel(const float *__restrict__ wts, int k,
+// slot adds nothing (a is already an f16 value).  PLAN false: one token, slot
+// s's row is row s.
+template <bool PLAN>
+__global__ void __launch_bounds__(256) moe_reduce_f16_kernel(const int32_t *__restrict__ ids,
+                                                             const float *__restrict__ wts, int k, int ne,
                                                              int64_t n_embd, MoeWs w,
                                                              _Float16 *__restrict__ out) {
     const int64_t t = blockIdx.y;
@@ -409,7 +413,9 @@ __global__ void __launch_bounds__(256) moe_reduce_f16_kernel(const float *__rest
     if (j >= n_embd) return;
     float a = 0.0f;
     for (int s = 0; s < k; s++) {
-        const int pos = w.plan_pos[t * k + s];
+        int pos;
+        if constexpr (PLAN) pos = w.plan_pos[t * k + s];
+        else pos = ids[s] >= 0 && ids[s] < ne ? s : -1;
         if (pos < 0) continue;
         const float vf = static_cast<float>(static_cast<_Float16>(w.part[static_cast<int64_t>(pos) * n_embd + j]));
         const float part = __fmul_rn(wts[t * k + s], __fmul_rn(vf, w.rscale[pos]));
@@ -695,6 +701,31 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
                            a.n_embd, w, static_cast<float *>(a.out));
         return hipGetLastError();
     }
+    if (a.act_f16 && a.n_tok == 1 && a.wt == DT_Q4_K && (a.wt_down == DT_Q4_K || a.wt_down == DT_Q6_K) &&
+        a.aligned16 && a.rb_gate == a.rb_up && a.k <= kMaxSegs) {
+        // one token: no plan; the streaming GEMV's routed gate/up, each slot's
+        // row scaled, its down projection slot by slot, the ordered reduce
+        // (128 experts, 4096 / 1536, top 8: 65 us through the rows kernel,
+        // 38 us here)
+        SegTable dn = d;
+        dn.n_in = static_cast<int>(a.n_ff);
+        dn.moe_down = 0;
+        dn.moe_slots = 1;
+        dn.seg[0].x = w.midf;
+        dn.seg[0].out = w.part;
+        if (gemv_stream_ok(DT_Q4_K, gu) && gemv_stream_ok(a.wt_down, dn)) {
+            hipError_t e = gemv_stream(DT_Q4_K, true, gu, st);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(moe_scale_kernel<false>, dim3(static_cast<unsigned>(a.k)), dim3(256), 0, st, a.n_ff,
+                               a.n_expert, w);
+            e = gemv_stream(a.wt_down, true, dn, st);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(moe_reduce_f16_kernel<false>, dim3(static_cast<unsigned>((a.n_embd + 255) / 256), 1),
+                               dim3(256), 0, st, a.ids, a.wts, a.k, a.n_expert, a.n_embd, w,
+                               static_cast<_Float16 *>(a.out));
+            return hipGetLastError();
+        }
+    }
     if (moe_rows(a)) {
         // plan; the tokens' rows prepared; gate/up of every active expert into
         // mid; (f16: each mid row scaled and rounded) the mid rows prepared;
@@ -719,7 +750,7 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
         if (e != hipSuccess) return e;
         uint8_t *prep2 = w.prep + al(gemm_rows_prep_bytes(a.n_tok, a.n_embd, planes, false));
         if (a.act_f16)
-            hipLaunchKernelGGL(moe_scale_kernel, dim3(static_cast<unsigned>(P)), dim3(256), 0, st, a.n_ff,
+            hipLaunchKernelGGL(moe_scale_kernel<true>, dim3(static_cast<unsigned>(P)), dim3(256), 0, st, a.n_ff,
                                a.n_expert, w);
         e = gemm_rows_prep(a.wt_down, a.act_f16 ? static_cast<const void *>(w.midf) : w.mid, a.act_f16, a.n_ff, P, a.n_ff,
                            planes, false, w.off + a.n_expert, prep2, r, st);
@@ -732,7 +763,7 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
         if (e != hipSuccess) return e;
         const dim3 rgrid(static_cast<unsigned>((a.n_embd + 255) / 256), static_cast<unsigned>(a.n_tok));
         if (a.act_f16)
-            hipLaunchKernelGGL(moe_reduce_f16_kernel, rgrid, dim3(256), 0, st, a.wts, a.k, a.n_embd, w,
+            hipLaunchKernelGGL(moe_reduce_f16_kernel<true>, rgrid, dim3(256), 0, st, a.ids, a.wts, a.k, a.n_expert, a.n_embd, w,
                                static_cast<_Float16 *>(a.out));
         else
             hipLaunchKernelGGL((moe_reduce_kernel<float>), rgrid, dim3(256), 0, st, a.ids, a.wts, a.k,
@@ -817,11 +848,11 @@ hipError_t moe_dispatch(const MoeArgs &a, void *ws, size_t ws_bytes, hipStream_t
     if (a.act_f16) {
         hipLaunchKernelGGL((moe_gu_kernel<_Float16, 2, 4>), cap(amax * ggu, wgu), dim3(64 * wgu), 0, st,
                            tab, static_cast<const _Float16 *>(a.xn), a.n_embd, a.n_ff, ggu, w);
-        hipLaunchKernelGGL(moe_scale_kernel, dim3(static_cast<unsigned>(P)), dim3(256), 0, st, a.n_ff,
+        hipLaunchKernelGGL(moe_scale_kernel<true>, dim3(static_cast<unsigned>(P)), dim3(256), 0, st, a.n_ff,
                            a.n_expert, w);
         hipLaunchKernelGGL((moe_down_kernel<_Float16, 2, 4>), cap(amax * gdn, wdn), dim3(64 * wdn), 0, st, tab,
                            a.n_embd, a.n_ff, gdn, w);
-        hipLaunchKernelGGL(moe_reduce_f16_kernel, rgrid, dim3(256), 0, st, a.wts, a.k, a.n_embd, w,
+        hipLaunchKernelGGL(moe_reduce_f16_kernel<true>, rgrid, dim3(256), 0, st, a.ids, a.wts, a.k, a.n_expert, a.n_embd, w,
                            static_cast<_Float16 *>(a.out));
         return hipGetLastError();
     }
