@@ -222,3 +222,41 @@ def test_rows_moe_f32(krk, torch_cuda, be32, dt, n_tok):
                     [mats[2, e] for e in range(ne)], dt, ids, wts, n_ff)
     for t in range(n_tok):
         assert rel(host(out)[t], ref[t]) <= GEMV_TOL, t
+
+
+@pytest.mark.parametrize("act", ["f32", "f16"])
+@pytest.mark.parametrize("n_tok", [1, 3, 700])
+def test_moe_plan_reduce_edges(krk, torch_cuda, be32, be16, act, n_tok):
+    """The plan over 300 experts (threads past the experts, 700 tokens: ids past
+    the ones kept in LDS) and the reduces: each token's row where the output
+    starts off a vector boundary is the aligned call's, bit for bit."""
+    torch = torch_cuda
+    be = be32 if act == "f32" else be16
+    td = torch.float32 if act == "f32" else torch.float16
+    ne, n_embd, n_ff, k = 300, 256, 256, 6
+    mats, table, keep = build_moe(krk, torch, O.Q4_K, ne, n_embd, n_ff, seed=2100)
+    ids, wts = O.router_topk(O.router_softmax(krk.synth_normal(n_tok * ne, seed=191).reshape(n_tok, ne)), k)
+    x = torch.from_numpy(krk.synth_normal(n_tok * n_embd, seed=192).reshape(n_tok, n_embd)).to("cuda", td)
+    d_ids, d_wts = dev(torch, ids), dev(torch, wts)
+    outs = []
+    say("moe plan", act, n_tok)
+    be.set_gemm_path(krk.PATH_EXACT)
+    try:
+        for off in (0, 1):
+            buf = torch.full((n_tok * n_embd + 8,), float("nan"), dtype=td, device="cuda")
+            out = buf[off:off + n_tok * n_embd]
+            be.moe_dispatch(table, 0, ne, d_ids, d_wts, x, out, n_tok, n_embd, n_ff, k)
+            be.sync()
+            assert torch.isnan(buf[:off]).all() and torch.isnan(buf[off + n_tok * n_embd:]).all()
+            outs.append(host(out).reshape(n_tok, n_embd))
+    finally:
+        be.set_gemm_path(krk.PATH_AUTO)
+        be.moe_table_forget(table)
+    assert np.array_equal(outs[0], outs[1])
+    sel = sorted({0, n_tok // 2, n_tok - 1})
+    ref = O.moe_ffn(host(x).astype(np.float32)[sel], [mats[0, e] for e in range(ne)], [mats[1, e] for e in range(ne)],
+                    [mats[2, e] for e in range(ne)], O.Q4_K, ids[sel], wts[sel], n_ff)
+    for i, t in enumerate(sel):
+        # f16: the slots' running sum is rounded to f16 k times (2^-11 each)
+        bar = GEMV_TOL if act == "f32" else GEMV_TOL + (k + 2) * 2.0**-11
+        assert rel(outs[0][t], ref[i]) <= bar, t
