@@ -428,6 +428,28 @@ int gemm_impl(krk_backend *b, void *out, const void *x, const void *w, int wt, i
     return e == hipSuccess ? KRK_OK : hip_fail(b, e, "mfma gemm");
 }
 
+// Groups of 9..128 rows whose matrices would each take the weight-streaming
+// GEMM (gemm_mfma), of one type and one x: in one launch.  A stream that is
+// being captured cannot grow the workspace; then the matrices run one by one.
+bool group_mfma(krk_backend *b, const void *const w[], int wt, const int64_t n_out[], int64_t n_in,
+                int n, int64_t rows, const void *const xs[], bool uniform) {
+    if (!uniform || n < 2 || rows <= kRowsExact || (b->path != KRK_PATH_AUTO && b->path != KRK_PATH_MFMA)) return false;
+    if (!krk::gemm_mfma_group_ok(wt, rows, n_out, n, n_in)) return false;
+    for (int m = 0; m < n; m++)
+        if ((xs && xs[m] != xs[0]) || rows_path(b, wt, n_out[m], n_in, rows, w[m])) return false;
+    if (krk::gemm_mfma_group_workspace(rows, n_out, n, n_in) <= b->ws_bytes) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(b->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+}
+
+int run_mfma_group(krk_backend *b, void *const out[], const void *x, const void *const w[], int wt,
+                   const int64_t n_out[], int64_t n_in, int n, int64_t rows) {
+    if (int s = ensure_ws(b, krk::gemm_mfma_group_workspace(rows, n_out, n, n_in))) return s;
+    const hipError_t e = krk::gemm_mfma_group(wt, w, krk_dtype_row_bytes(wt, n_in), x, b->act == KRK_ACT_F16, out,
+                                              rows, n_out, n, n_in, b->ws, b->ws_bytes, b->stream);
+    return e == hipSuccess ? KRK_OK : hip_fail(b, e, "mfma gemm");
+}
+
 }  // namespace
 
 extern "C" {
@@ -489,6 +511,8 @@ int krk_gemm_group(krk_backend *b, void *const out[], const void *x, const void 
             one = (!xs || xs[m] == xs[0]) && rows_path(b, t0, n_out[m], n_in, rows, w[m]);
         one = one && krk::gemm_rows_tiles_ok(t0, n_in, n_out, n_mat, b->tile_cnt != nullptr);
         if (one) return run_rows(b, out, xs ? xs[0] : x, w, t0, n_out, n_in, n_mat, rows, nullptr, 0);
+        if (group_mfma(b, w, t0, n_out, n_in, n_mat, rows, xs, uniform))
+            return run_mfma_group(b, out, xs ? xs[0] : x, w, t0, n_out, n_in, n_mat, rows);
         for (int m = 0; m < n_mat; m++)
             if (int s = krk_gemm(b, out[m], xs ? xs[m] : x, w[m], wts ? wts[m] : wt, n_out[m], n_in,
                                  rows))

@@ -170,6 +170,13 @@ constexpr int kTileCounters = 4096;
 hipError_t gemm_mfma(int dt, const void *w, int64_t row_bytes, const void *x, bool act_f16,
                      void *out, int64_t M, int64_t N, int64_t K, void *ws, size_t ws_bytes,
                      unsigned *cnt, hipStream_t st);
+// n matrices of one type against the same rows in one launch (batches that
+// take the weight-streaming kernel)
+bool gemm_mfma_group_ok(int dt, int64_t M, const int64_t N[], int n, int64_t K);
+size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K);
+hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, const void *x, bool act_f16,
+                           void *const out[], int64_t M, const int64_t N[], int n, int64_t K, void *ws,
+                           size_t ws_bytes, hipStream_t st);
 // Grouped expert GEMM on the f16 MFMA: one launch per projection over the
 // MoE plan's items {expert, first plan position, rows <= 32 mi, 0}; X holds
 // f16 activation rows in plan order [P, K].  Gate/up: out = f16 rows
@@ -188,9 +195,10 @@ struct MoeGemmArgs {
     int max_items;             // items the grid covers (an upper bound)
     int mi;                    // item rows = 32 mi, mi in {1, 2}
     bool gate_up;
-    // dense mode (w non-null, items unused, not gate/up): one weight matrix,
-    // items of 32 mi of the M rows of X, out [M, N] in f32 or f16
-    const void *w;
+    // dense mode (n_seg > 0, items unused, not gate/up): n_seg weight matrices,
+    // items of 32 mi of the M rows of X, each matrix's out [M, N] in f32 or f16
+    struct Seg { const void *w; void *out; int N; } seg[kMaxSegs];
+    int n_seg;
     int M;
     bool out_f16;
     int ksplit;                // dense: K in ksplit whole-block ranges, f32 partials [ksplit][M][N] at out

@@ -260,3 +260,27 @@ def test_moe_plan_reduce_edges(krk, torch_cuda, be32, be16, act, n_tok):
         # f16: the slots' running sum is rounded to f16 k times (2^-11 each)
         bar = GEMV_TOL if act == "f32" else GEMV_TOL + (k + 2) * 2.0**-11
         assert rel(outs[0][t], ref[i]) <= bar, t
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("rows,act,n_in", [(33, "f32", 256), (41, "f16", 4096), (128, "f32", 2304)])
+def test_mfma_group(krk, torch_cuda, be32, be16, dt, rows, act, n_in):
+    """A group of 9..128 rows in one launch, one and several K ranges, matrices
+    that end inside a tile and of one row: the MFMA GEMM bar, and one gemm each."""
+    torch = torch_cuda
+    be, td = (be32, torch.float32) if act == "f32" else (be16, torch.float16)
+    shapes = [300, 1, 1025]
+    ws = [dev(torch, make_weights(krk, dt, n, n_in, seed=2200 + i)) for i, n in enumerate(shapes)]
+    x = torch.from_numpy(krk.synth_normal(rows * n_in, seed=2204).reshape(rows, n_in)).to("cuda", td)
+    say("mfma group", dt, rows, act, n_in)
+    outs = [torch.full((rows, n), float("nan"), dtype=td, device="cuda") for n in shapes]
+    assert be.gemm_group(outs, x, ws, dt, shapes, n_in, rows) == (False, False)
+    be.sync()
+    first = [host(o).copy() for o in outs]
+    for o, w, n in zip(first, ws, shapes):
+        assert rel(o, O.gemm(dt, host(w), host(x).astype(np.float32), n)) <= GEMM_TOL
+        one = torch.full((rows, n), float("nan"), dtype=td, device="cuda")
+        be.gemm(one, x, w, dt, n, n_in, rows)
+        be.sync()
+        # the same products; K in other ranges, summed in f32
+        assert rel(o, host(one)) <= (1e-6 if act == "f32" else 2.0**-10)
