@@ -437,14 +437,14 @@ bool group_mfma(krk_backend *b, const void *const w[], int wt, const int64_t n_o
     if (!krk::gemm_mfma_group_ok(wt, rows, n_out, n, n_in)) return false;
     for (int m = 0; m < n; m++)
         if ((xs && xs[m] != xs[0]) || rows_path(b, wt, n_out[m], n_in, rows, w[m])) return false;
-    if (krk::gemm_mfma_group_workspace(rows, n_out, n, n_in) <= b->ws_bytes) return true;
+    if (krk::gemm_mfma_group_workspace(rows, n_out, n, n_in, false) <= b->ws_bytes) return true;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     return hipStreamIsCapturing(b->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
 }
 
 int run_mfma_group(krk_backend *b, void *const out[], const void *x, const void *const w[], int wt,
                    const int64_t n_out[], int64_t n_in, int n, int64_t rows) {
-    if (int s = ensure_ws(b, krk::gemm_mfma_group_workspace(rows, n_out, n, n_in))) return s;
+    if (int s = ensure_ws(b, krk::gemm_mfma_group_workspace(rows, n_out, n, n_in, false))) return s;
     const hipError_t e = krk::gemm_mfma_group(wt, w, krk_dtype_row_bytes(wt, n_in), x, b->act == KRK_ACT_F16, out,
                                               rows, n_out, n, n_in, b->ws, b->ws_bytes, b->stream);
     return e == hipSuccess ? KRK_OK : hip_fail(b, e, "mfma gemm");

@@ -923,24 +923,35 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(SplitSum a, int spli
     }
 }
 
-static int pick_split(int64_t M, int64_t N, int64_t K, int dt) {
+// K values of each of s ranges, whole blocks (the last range may be shorter)
+static int64_t split_range(int64_t K, int64_t s, int64_t kblk) { return (K / kblk + s - 1) / s * kblk; }
+
+// even: only splits into equal ranges (what a fixed scratch is asked for)
+static int pick_split(int64_t M, int64_t N, int64_t K, int dt, bool even) {
     const int64_t tiles = ((M + GB_M - 1) / GB_M) * ((N + GB_N - 1) / GB_N);
     const int64_t kblk = blk_vals(dt) < GB_K ? GB_K : blk_vals(dt);
     const int64_t cus = device_cus();
     // Estimated time of a split (us): rounds of resident workgroups x K per
     // split at ~0.034 us per K value and round (a 256 x 256 tile, measured),
     // plus the partials' traffic -- written and read back, 8 s M N bytes --
-    // at ~4 TB/s.  Splits keep at least 1024 K in whole blocks; ties keep
-    // the smaller split.
-    auto cost = [&](int64_t s) {
+    // at ~4 TB/s, plus the reduce launch past two splits.  Ranges keep at
+    // least 256 K in whole blocks; ties keep the smaller split.  Ranges may
+    // differ in length: 11008 -> 4096 (43 blocks), 256 f16 rows of Q4_K 281 ->
+    // 53 us, 512 f32 rows of Q6_K 955 -> 121; at least 1024 K a range left a
+    // small matrix on a few CUs: 4864 -> 2048, 300 rows of Q8_0, 74 -> 41.
+    auto cost = [&](int64_t s, int64_t range) {
         const double rounds = static_cast<double>((tiles * s + cus - 1) / cus);
         const double part = s > 1 ? 8.0 * static_cast<double>(s) * M * N / 4.0e6 : 0.0;
-        return rounds * static_cast<double>(K / s) * 0.034 + part;
+        return rounds * static_cast<double>(range) * 0.034 + part + (s > 2 ? 4.0 : 0.0);
     };
     int best = 1;
-    double best_cost = cost(1);
-    for (int s = 2; s <= 64 && K / s >= 1024 && K % s == 0 && (K / s) % kblk == 0; s *= 2) {
-        const double c = cost(s);
+    double best_cost = cost(1, K);
+    if (K % kblk) return best;
+    for (int s = 2; s <= 64; s++) {
+        const int64_t r = split_range(K, s, kblk);
+        if (r < (even ? 1024 : 256)) break;
+        if (even ? (s & (s - 1)) != 0 || r * s != K : (s - 1) * r >= K) continue;
+        const double c = cost(s, r);
         if (c < best_cost) {
             best_cost = c;
             best = s;
@@ -957,18 +968,27 @@ static bool stream_gemm(int dt, int64_t M, int64_t N, int64_t K) {
     return M <= kStreamGemmRows && K % 256 == 0 && N < (1LL << 31) && K < (1LL << 31) && moe_gemm_ok(dt);
 }
 
-// K ranges of a dense streaming launch: the largest divisor of the block
-// count up to what brings the workgroups to one per CU (two per CU measured
-// slower from 9 to 64 rows: 16 rows 17.8 -> 19.4 us up, 20.8 -> 24.6 down)
-static int stream_split(int64_t M, const int64_t N[], int n, int64_t K) {
+// K ranges of a dense streaming launch: the fewest that give the least rounds
+// of workgroups x blocks per range, at one workgroup per CU (two per CU
+// measured slower from 9 to 64 rows: 16 rows 17.8 -> 19.4 us up, 20.8 -> 24.6
+// down).  The last range may be shorter: 43 blocks (a K of 11008), which only
+// 1 and 43 divide, in 15 ranges: 20 f16 rows of Q4_K 108 -> 21 us.  even: equal ranges only, the largest divisor of
+// the block count up to one workgroup per CU (what a fixed scratch is asked for).
+static int stream_split(int64_t M, const int64_t N[], int n, int64_t K, bool even) {
     const int64_t mt = M <= 32 ? 32 : 64;
     int64_t wgs = 0;
     for (int m = 0; m < n; m++) wgs += ((M + mt - 1) / mt) * ((N[m] + 255) / 256);
-    const int64_t want = (device_cus() + wgs - 1) / wgs;
+    const int64_t cus = device_cus(), want = (cus + wgs - 1) / wgs;
     const int64_t nb = K / 256;
     int best = 1;
-    for (int s = 1; s <= nb && s <= want; s++)
-        if (nb % s == 0) best = s;
+    int64_t best_cost = 0;
+    for (int s = 1; s <= nb && s <= want; s++) {
+        const int64_t r = (nb + s - 1) / s, c = (wgs * s + cus - 1) / cus * r;
+        if (even ? nb % s == 0 : (s - 1) * r < nb && (s == 1 || c < best_cost)) {
+            best = s;
+            best_cost = c;
+        }
+    }
     return best;
 }
 static size_t al256(size_t v) { return (v + 255) & ~size_t(255); }
@@ -1004,16 +1024,19 @@ bool gemm_mfma_group_ok(int dt, int64_t M, const int64_t N[], int n, int64_t K) 
 }
 
 // f32 rows as f16, and the split partials
-size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K) {
-    const int s = stream_split(M, N, n, K);
+size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool minimal) {
+    const int s = stream_split(M, N, n, K, minimal);
     size_t b = al256(static_cast<size_t>(M * K) * sizeof(_Float16));
-    for (int m = 0; m < n && s > 1; m++) b += al256(static_cast<size_t>(s) * M * N[m] * sizeof(float));
+    for (int m = 0; m < n && s > 1; m++) {
+        const size_t p = static_cast<size_t>(s) * M * N[m] * sizeof(float);
+        b += m + 1 < n ? al256(p) : p;
+    }
     return b;
 }
 
 size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal) {
-    if (stream_gemm(dt, M, N, K)) return gemm_mfma_group_workspace(M, &N, 1, K);
-    const int s = pick_split(M, N, K, dt);
+    if (stream_gemm(dt, M, N, K)) return gemm_mfma_group_workspace(M, &N, 1, K, minimal);
+    const int s = pick_split(M, N, K, dt, minimal);
     const size_t flat = splitk_floats(M, N, s, false), imgs = splitk_floats(M, N, s, true);
     const size_t part = (minimal || flat > imgs ? flat : imgs) * sizeof(float);
     return minimal || act_f16 || !rows_once(dt) ? part : al256(part) + static_cast<size_t>(M * K) * sizeof(_Float16);
@@ -1025,8 +1048,9 @@ static hipError_t launch_f16(const void *w, int64_t rb, const void *x, void *out
                              hipStream_t st) {
     const int tiles_m = static_cast<int>((M + GB_M - 1) / GB_M);
     const int tiles_n = static_cast<int>((N + GB_N - 1) / GB_N);
-    const int s = pick_split(M, N, K, DT);
-    const int kps = static_cast<int>(K / s);
+    int s = pick_split(M, N, K, DT, false);
+    if (ws_bytes < splitk_floats(M, N, s, false) * sizeof(float)) s = pick_split(M, N, K, DT, true);
+    const int kps = static_cast<int>(s > 1 ? split_range(K, s, blk_vals(DT) < GB_K ? GB_K : blk_vals(DT)) : K);
     float *part = nullptr;
     if (s > 1) {
         if (ws_bytes < splitk_floats(M, N, s, false) * sizeof(float)) return hipErrorInvalidValue;
@@ -1061,9 +1085,9 @@ static hipError_t launch_f16(const void *w, int64_t rb, const void *x, void *out
 hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, const void *x, bool act_f16,
                            void *const out[], int64_t M, const int64_t N[], int n, int64_t K, void *ws,
                            size_t ws_bytes, hipStream_t st) {
-    if (!gemm_mfma_group_ok(dt, M, N, n, K) || ws_bytes < gemm_mfma_group_workspace(M, N, n, K))
+    if (!gemm_mfma_group_ok(dt, M, N, n, K) || ws_bytes < gemm_mfma_group_workspace(M, N, n, K, true))
         return hipErrorInvalidValue;
-    const int split = stream_split(M, N, n, K);
+    const int split = stream_split(M, N, n, K, ws_bytes < gemm_mfma_group_workspace(M, N, n, K, false));
     uint8_t *part = static_cast<uint8_t *>(ws) + al256(static_cast<size_t>(M * K) * sizeof(_Float16));
     MoeGemmArgs g{};
     g.x = x;
@@ -1084,6 +1108,7 @@ hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, con
     }
     g.n_seg = n;
     g.ksplit = split;
+    g.krange = static_cast<int>((K / 256 + split - 1) / split);
     g.out_f16 = act_f16;
     g.row_bytes = row_bytes;
     g.K = static_cast<int>(K);
@@ -1373,8 +1398,8 @@ __global__ void __launch_bounds__(MG_THREADS) __attribute__((amdgpu_waves_per_eu
         wrow[c] = wb + static_cast<int64_t>(row[c] < N ? row[c] : N - 1) * a.row_bytes;
     }
     // a dense launch's K range: its blocks start kb0 blocks into every row
-    const int nblk = a.K / 256 / (dense ? a.ksplit : 1);
-    const int64_t kb0 = static_cast<int64_t>(ks) * nblk;
+    const int64_t kb0 = dense ? static_cast<int64_t>(ks) * a.krange : 0;
+    const int nblk = dense ? min(a.krange, a.K / 256 - static_cast<int>(kb0)) : a.K / 256;
     if (ks) {
         const int64_t bb = a.row_bytes / (a.K / 256);   // bytes per 256 values
 #pragma unroll
@@ -1557,7 +1582,8 @@ template <int DT, bool GU>
 static hipError_t launch_moe_gemm(const MoeGemmArgs &a, hipStream_t st) {
     const bool dense = a.n_seg > 0;
     if (a.K % 256 || (!dense && a.N <= 0) || a.n_seg > kMaxSegs ||
-        (dense ? (GU || a.M <= 0 || a.ksplit < 1 || (a.K / 256) % a.ksplit) : a.max_items <= 0))
+        (dense ? (GU || a.M <= 0 || a.ksplit < 1 || a.krange < 1 || (a.ksplit - 1) * a.krange >= a.K / 256 ||
+                  a.ksplit * a.krange < a.K / 256) : a.max_items <= 0))
         return hipErrorInvalidValue;
     int ntiles = dense ? 0 : (a.N + (GU ? 127 : 255)) / (GU ? 128 : 256);
     for (int m = 0; m < a.n_seg; m++) ntiles += (a.seg[m].N + 255) / 256;

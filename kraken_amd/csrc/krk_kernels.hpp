@@ -157,8 +157,8 @@ hipError_t quantize_q8_rows_f16codes(const void *x, bool x_f16, int64_t rows, in
 
 // Prefill GEMM (f16 MFMA, f32 accumulate) and the Q8_0 x Q8 int8 MFMA rung.
 // out[M, N] = X[M, K] . deq(W)[N, K]^T.  `ws` is device scratch of ws_bytes.
-// scratch of gemm_mfma: what its fastest form needs, or (minimal) the
-// least it runs with
+// scratch of gemm_mfma: what its fastest form needs, or (minimal) what a
+// fixed scratch has to hold: K ranges of equal length only, f32 staging
 size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal);
 // compute units of the current device (cached on first use)
 int device_cus();
@@ -173,7 +173,7 @@ hipError_t gemm_mfma(int dt, const void *w, int64_t row_bytes, const void *x, bo
 // n matrices of one type against the same rows in one launch (batches that
 // take the weight-streaming kernel)
 bool gemm_mfma_group_ok(int dt, int64_t M, const int64_t N[], int n, int64_t K);
-size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K);
+size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool minimal);
 hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, const void *x, bool act_f16,
                            void *const out[], int64_t M, const int64_t N[], int n, int64_t K, void *ws,
                            size_t ws_bytes, hipStream_t st);
@@ -201,7 +201,8 @@ struct MoeGemmArgs {
     int n_seg;
     int M;
     bool out_f16;
-    int ksplit;                // dense: K in ksplit whole-block ranges, f32 partials [ksplit][M][N] at out
+    int ksplit;                // dense: K in ksplit ranges of krange blocks (the last may be shorter), f32
+    int krange;                // partials [ksplit][M][N] at out
     const int32_t *xtok;       // non-null: plan position p's activation row is x row xtok[p] (gate/up on
                                // the tokens' rows); null: x rows in plan order
 };

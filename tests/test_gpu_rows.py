@@ -284,3 +284,26 @@ def test_mfma_group(krk, torch_cuda, be32, be16, dt, rows, act, n_in):
         be.sync()
         # the same products; K in other ranges, summed in f32
         assert rel(o, host(one)) <= (1e-6 if act == "f32" else 2.0**-10)
+
+
+@pytest.mark.parametrize("dt", TYPES)
+@pytest.mark.parametrize("rows,n_out,n_in", [(33, 300, 2816), (160, 300, 2816), (257, 520, 3328), (512, 4096, 11008)])
+def test_uneven_k_ranges(krk, torch_cuda, be32, dt, rows, n_out, n_in):
+    """K ranges of unequal length (block counts of 11, 13 and 43, prime), on
+    the weight-streaming and the tile GEMM, replayed into the same workspace,
+    and with the fixed scratch (which does not hold the last shape's ranges)."""
+    torch = torch_cuda
+    w = dev(torch, make_weights(krk, dt, n_out, n_in, seed=2300))
+    x = dev(torch, krk.synth_normal(rows * n_in, seed=2301).reshape(rows, n_in))
+    say("uneven ranges", dt, rows, n_out, n_in)
+    outs = []
+    for call in (be32.gemm, be32.gemm, be32.gemm_noalloc):
+        out = torch.full((rows, n_out), float("nan"), dtype=torch.float32, device="cuda")
+        call(out, x, w, dt, n_out, n_in, rows)
+        be32.sync()
+        outs.append(host(out).copy())
+    sel = [0, rows // 2, rows - 1]
+    ref = O.gemm(dt, host(w), host(x)[sel], n_out)
+    assert rel(outs[0][sel], ref) <= GEMM_TOL
+    assert np.array_equal(outs[0], outs[1])
+    assert rel(outs[2], outs[0]) <= 1e-6   # (the same products; the ranges, and with them the order of the sums)
