@@ -29,6 +29,7 @@
 // with the host rule (quantize_q8_32_d), v_mfma_i32_32x32x32_i8 per 32-value
 // block, and the block fold acc = fma((f32)isum, d_w * d_x, acc) of
 // dot_q8_0_q8_scalar (src/quant.cpp:3261-3279).
+#include <algorithm>
 #include <type_traits>
 
 #include "krk_formats.hpp"
@@ -926,7 +927,11 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(SplitSum a, int spli
 // K values of each of s ranges, whole blocks (the last range may be shorter)
 static int64_t split_range(int64_t K, int64_t s, int64_t kblk) { return (K / kblk + s - 1) / s * kblk; }
 
-// even: only splits into equal ranges (what a fixed scratch is asked for)
+// Ranges of unequal length, or of less than 1024 K, are taken only where their
+// partials fit kSplitScratch, the size of the caller's fixed scratch: the split
+// does not depend on which scratch a call has (the results would), and a call
+// that had room keeps it.  even: without those.
+constexpr size_t kSplitScratch = size_t(64) << 20;
 static int pick_split(int64_t M, int64_t N, int64_t K, int dt, bool even) {
     const int64_t tiles = ((M + GB_M - 1) / GB_M) * ((N + GB_N - 1) / GB_N);
     const int64_t kblk = blk_vals(dt) < GB_K ? GB_K : blk_vals(dt);
@@ -949,8 +954,9 @@ static int pick_split(int64_t M, int64_t N, int64_t K, int dt, bool even) {
     if (K % kblk) return best;
     for (int s = 2; s <= 64; s++) {
         const int64_t r = split_range(K, s, kblk);
-        if (r < (even ? 1024 : 256)) break;
-        if (even ? (s & (s - 1)) != 0 || r * s != K : (s - 1) * r >= K) continue;
+        if (r < 256) break;
+        const bool eq = r >= 1024 && (s & (s - 1)) == 0 && r * s == K;
+        if (!eq && (even || (s - 1) * r >= K || static_cast<size_t>(s) * M * N * sizeof(float) > kSplitScratch)) continue;
         const double c = cost(s, r);
         if (c < best_cost) {
             best_cost = c;
@@ -972,19 +978,25 @@ static bool stream_gemm(int dt, int64_t M, int64_t N, int64_t K) {
 // of workgroups x blocks per range, at one workgroup per CU (two per CU
 // measured slower from 9 to 64 rows: 16 rows 17.8 -> 19.4 us up, 20.8 -> 24.6
 // down).  The last range may be shorter: 43 blocks (a K of 11008), which only
-// 1 and 43 divide, in 15 ranges: 20 f16 rows of Q4_K 108 -> 21 us.  even: equal ranges only, the largest divisor of
-// the block count up to one workgroup per CU (what a fixed scratch is asked for).
+// 1 and 43 divide, in 15 ranges: 20 f16 rows of Q4_K 108 -> 21 us.  Unequal
+// ranges only within kSplitScratch; even: equal ones, the largest divisor of
+// the block count up to one workgroup per CU.
 static int stream_split(int64_t M, const int64_t N[], int n, int64_t K, bool even) {
     const int64_t mt = M <= 32 ? 32 : 64;
     int64_t wgs = 0;
     for (int m = 0; m < n; m++) wgs += ((M + mt - 1) / mt) * ((N[m] + 255) / 256);
     const int64_t cus = device_cus(), want = (cus + wgs - 1) / wgs;
     const int64_t nb = K / 256;
+    auto fits = [&](int s) {
+        double b = 2.0 * M * K;
+        for (int m = 0; m < n; m++) b += 4.0 * s * M * N[m] + 256;
+        return b <= static_cast<double>(kSplitScratch);
+    };
     int best = 1;
     int64_t best_cost = 0;
     for (int s = 1; s <= nb && s <= want; s++) {
         const int64_t r = (nb + s - 1) / s, c = (wgs * s + cus - 1) / cus * r;
-        if (even ? nb % s == 0 : (s - 1) * r < nb && (s == 1 || c < best_cost)) {
+        if (even ? nb % s == 0 : (s - 1) * r < nb && (s == 1 || c < best_cost) && (nb % s == 0 || fits(s))) {
             best = s;
             best_cost = c;
         }
@@ -1024,8 +1036,8 @@ bool gemm_mfma_group_ok(int dt, int64_t M, const int64_t N[], int n, int64_t K) 
 }
 
 // f32 rows as f16, and the split partials
-size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool minimal) {
-    const int s = stream_split(M, N, n, K, minimal);
+size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool even) {
+    const int s = stream_split(M, N, n, K, even);
     size_t b = al256(static_cast<size_t>(M * K) * sizeof(_Float16));
     for (int m = 0; m < n && s > 1; m++) {
         const size_t p = static_cast<size_t>(s) * M * N[m] * sizeof(float);
@@ -1035,9 +1047,14 @@ size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K,
 }
 
 size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal) {
-    if (stream_gemm(dt, M, N, K)) return gemm_mfma_group_workspace(M, &N, 1, K, minimal);
-    const int s = pick_split(M, N, K, dt, minimal);
-    const size_t flat = splitk_floats(M, N, s, false), imgs = splitk_floats(M, N, s, true);
+    // (minimal: no less than equal ranges would need, which a fixed scratch
+    // has always been asked for)
+    if (stream_gemm(dt, M, N, K))
+        return std::max(gemm_mfma_group_workspace(M, &N, 1, K, false),
+                        minimal ? gemm_mfma_group_workspace(M, &N, 1, K, true) : 0);
+    const int s = pick_split(M, N, K, dt, false);
+    const size_t even = minimal ? splitk_floats(M, N, pick_split(M, N, K, dt, true), false) : 0;
+    const size_t flat = std::max(splitk_floats(M, N, s, false), even), imgs = splitk_floats(M, N, s, true);
     const size_t part = (minimal || flat > imgs ? flat : imgs) * sizeof(float);
     return minimal || act_f16 || !rows_once(dt) ? part : al256(part) + static_cast<size_t>(M * K) * sizeof(_Float16);
 }
@@ -1048,8 +1065,7 @@ static hipError_t launch_f16(const void *w, int64_t rb, const void *x, void *out
                              hipStream_t st) {
     const int tiles_m = static_cast<int>((M + GB_M - 1) / GB_M);
     const int tiles_n = static_cast<int>((N + GB_N - 1) / GB_N);
-    int s = pick_split(M, N, K, DT, false);
-    if (ws_bytes < splitk_floats(M, N, s, false) * sizeof(float)) s = pick_split(M, N, K, DT, true);
+    const int s = pick_split(M, N, K, DT, false);
     const int kps = static_cast<int>(s > 1 ? split_range(K, s, blk_vals(DT) < GB_K ? GB_K : blk_vals(DT)) : K);
     float *part = nullptr;
     if (s > 1) {
@@ -1085,9 +1101,9 @@ static hipError_t launch_f16(const void *w, int64_t rb, const void *x, void *out
 hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, const void *x, bool act_f16,
                            void *const out[], int64_t M, const int64_t N[], int n, int64_t K, void *ws,
                            size_t ws_bytes, hipStream_t st) {
-    if (!gemm_mfma_group_ok(dt, M, N, n, K) || ws_bytes < gemm_mfma_group_workspace(M, N, n, K, true))
+    if (!gemm_mfma_group_ok(dt, M, N, n, K) || ws_bytes < gemm_mfma_group_workspace(M, N, n, K, false))
         return hipErrorInvalidValue;
-    const int split = stream_split(M, N, n, K, ws_bytes < gemm_mfma_group_workspace(M, N, n, K, false));
+    const int split = stream_split(M, N, n, K, false);
     uint8_t *part = static_cast<uint8_t *>(ws) + al256(static_cast<size_t>(M * K) * sizeof(_Float16));
     MoeGemmArgs g{};
     g.x = x;

@@ -158,7 +158,7 @@ hipError_t quantize_q8_rows_f16codes(const void *x, bool x_f16, int64_t rows, in
 // Prefill GEMM (f16 MFMA, f32 accumulate) and the Q8_0 x Q8 int8 MFMA rung.
 // out[M, N] = X[M, K] . deq(W)[N, K]^T.  `ws` is device scratch of ws_bytes.
 // scratch of gemm_mfma: what its fastest form needs, or (minimal) what a
-// fixed scratch has to hold: K ranges of equal length only, f32 staging
+// fixed scratch has to hold (f32 staging, the range sums by the reduce kernel)
 size_t gemm_mfma_workspace(int dt, bool act_f16, int64_t M, int64_t N, int64_t K, bool minimal);
 // compute units of the current device (cached on first use)
 int device_cus();
@@ -173,7 +173,7 @@ hipError_t gemm_mfma(int dt, const void *w, int64_t row_bytes, const void *x, bo
 // n matrices of one type against the same rows in one launch (batches that
 // take the weight-streaming kernel)
 bool gemm_mfma_group_ok(int dt, int64_t M, const int64_t N[], int n, int64_t K);
-size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool minimal);
+size_t gemm_mfma_group_workspace(int64_t M, const int64_t N[], int n, int64_t K, bool even);
 hipError_t gemm_mfma_group(int dt, const void *const w[], int64_t row_bytes, const void *x, bool act_f16,
                            void *const out[], int64_t M, const int64_t N[], int n, int64_t K, void *ws,
                            size_t ws_bytes, hipStream_t st);

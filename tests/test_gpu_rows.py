@@ -291,7 +291,8 @@ def test_mfma_group(krk, torch_cuda, be32, be16, dt, rows, act, n_in):
 def test_uneven_k_ranges(krk, torch_cuda, be32, dt, rows, n_out, n_in):
     """K ranges of unequal length (block counts of 11, 13 and 43, prime), on
     the weight-streaming and the tile GEMM, replayed into the same workspace,
-    and with the fixed scratch (which does not hold the last shape's ranges)."""
+    and with the fixed scratch, bit for bit (it does not hold the last shape's
+    ranges beside the rounded rows)."""
     torch = torch_cuda
     w = dev(torch, make_weights(krk, dt, n_out, n_in, seed=2300))
     x = dev(torch, krk.synth_normal(rows * n_in, seed=2301).reshape(rows, n_in))
@@ -305,5 +306,4 @@ def test_uneven_k_ranges(krk, torch_cuda, be32, dt, rows, n_out, n_in):
     sel = [0, rows // 2, rows - 1]
     ref = O.gemm(dt, host(w), host(x)[sel], n_out)
     assert rel(outs[0][sel], ref) <= GEMM_TOL
-    assert np.array_equal(outs[0], outs[1])
-    assert rel(outs[2], outs[0]) <= 1e-6   # (the same products; the ranges, and with them the order of the sums)
+    assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
