@@ -148,9 +148,12 @@ int krk_dtype_row_aligned(int wt, int64_t n);
  * rows == 1..8: fused dequant+dot GEMV with exact products and f32
  *               accumulation; Q4_K at rows == 1 forms the products on the
  *               int8 matrix cores from exact digit planes of x (rounded at
- *               2^-23 of each 32-value sub-block's maximum), and Q4_K at
- *               rows == 2..8 the same, the rows' digit tables built once per
- *               call in the handle's workspace (grown on the first such call).
+ *               2^-23 of each 32-value sub-block's maximum).  Several rows
+ *               of Q4_K, Q5_K, Q6_K, Q8_0 and Q4_0 form them on the f16
+ *               matrix cores from the weight codes, f32 rows as two f16
+ *               planes (22 bits below each row's maximum), or (Q4_K, up to
+ *               five rows) as one row does; the prepared rows lie in the
+ *               handle's workspace (grown on the first such call).
  * rows  > 8   : per krk_set_gemm_path. */
 int krk_gemm(krk_backend *b, void *out, const void *x, const void *w, int wt,
              int64_t n_out, int64_t n_in, int64_t rows);
@@ -159,7 +162,7 @@ int krk_gemm(krk_backend *b, void *out, const void *x, const void *w, int wt,
  * callers that cannot allocate device memory -- code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc.  Same
  * arguments, kernels and results as krk_gemm (bit-identical), but the
- * split-K partials, int8 activation codes and several-row digit tables that
+ * split-K partials, int8 activation codes and prepared rows that
  * krk_gemm keeps in the handle's growing workspace live in a fixed device array of
  * krk_gemm_noalloc_scratch_bytes() (64 MiB) instead: one per device, held
  * until the process ends, shared by every handle on that device.  The array
@@ -252,7 +255,8 @@ int krk_moe_plan_build(krk_backend *b, const void *ids, int64_t n_rows, int k,
  * or more whose banks are uniform Q4_K/Q5_K/Q6_K/Q8_0/Q4_0/MXFP4 (gate and
  * up of one type) form their products from f16 operands on the matrix
  * cores, as a gemm of more than 8 rows does, unless krk_set_gemm_path
- * selected KRK_PATH_EXACT.
+ * selected KRK_PATH_EXACT.  Scratch (the plan, the mid rows, the prepared rows)
+ * lies in the handle's workspace, grown on the first call that needs it.
  * The first call for a (table, layer, n_expert, n_embd, n_ff) reads that
  * layer's entries back once and validates every one: all three matrices
  * present, of a served type (types may vary from expert to expert and

@@ -337,16 +337,23 @@ bool rows_path(const krk_backend *b, int wt, int64_t n_out, int64_t n_in, int64_
            krk::gemm_rows_tiles_ok(wt, n_in, &n_out, 1, b->tile_cnt != nullptr);
 }
 
+int rows_planes(const krk_backend *b, int64_t rows) { return b->act != KRK_ACT_F16 && rows <= kRowsExact ? 2 : 1; }
+// its scratch: the prepared rows and the K ranges' partials
+size_t rows_scratch(const krk_backend *b, const int64_t n_out[], int64_t n_in, int n, int64_t rows) {
+    int64_t n_total = 0;
+    for (int m = 0; m < n; m++) n_total += n_out[m];
+    return krk::gemm_rows_prep_bytes(rows, n_in, rows_planes(b, rows), true) +
+           krk::gemm_rows_part_bytes(rows, n_total, n_in);
+}
+
 // n matrices of one type against the same rows: the rows prepared once, one
 // launch.  ws as in gemm_impl.
 int run_rows(krk_backend *b, void *const out[], const void *x, const void *const w[], int wt, const int64_t n_out[],
              int64_t n_in, int n, int64_t rows, void *ws, size_t ws_bytes) {
     const bool f16 = b->act == KRK_ACT_F16;
-    const int planes = !f16 && rows <= kRowsExact ? 2 : 1;
-    int64_t n_total = 0;
-    for (int m = 0; m < n; m++) n_total += n_out[m];
+    const int planes = rows_planes(b, rows);
     const size_t prep = krk::gemm_rows_prep_bytes(rows, n_in, planes, true);
-    const size_t need = prep + krk::gemm_rows_part_bytes(rows, n_total, n_in);
+    const size_t need = rows_scratch(b, n_out, n_in, n, rows);
     if (ws) {
         if (need > ws_bytes)
             return fail(b, KRK_ERR_NOMEM, "gemm rows need %zu bytes of scratch; the fixed scratch holds %zu", need,
@@ -428,18 +435,23 @@ int gemm_impl(krk_backend *b, void *out, const void *x, const void *w, int wt, i
     return e == hipSuccess ? KRK_OK : hip_fail(b, e, "mfma gemm");
 }
 
+// A stream that is being captured cannot grow the workspace: a group that
+// would need more than its matrices alone runs them one by one then.
+bool ws_ready(krk_backend *b, size_t need) {
+    if (need <= b->ws_bytes) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(b->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+}
+
 // Groups of 9..128 rows whose matrices would each take the weight-streaming
-// GEMM (gemm_mfma), of one type and one x: in one launch.  A stream that is
-// being captured cannot grow the workspace; then the matrices run one by one.
+// GEMM (gemm_mfma), of one type and one x: in one launch.
 bool group_mfma(krk_backend *b, const void *const w[], int wt, const int64_t n_out[], int64_t n_in,
                 int n, int64_t rows, const void *const xs[], bool uniform) {
     if (!uniform || n < 2 || rows <= kRowsExact || (b->path != KRK_PATH_AUTO && b->path != KRK_PATH_MFMA)) return false;
     if (!krk::gemm_mfma_group_ok(wt, rows, n_out, n, n_in)) return false;
     for (int m = 0; m < n; m++)
         if ((xs && xs[m] != xs[0]) || rows_path(b, wt, n_out[m], n_in, rows, w[m])) return false;
-    if (krk::gemm_mfma_group_workspace(rows, n_out, n, n_in, false) <= b->ws_bytes) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(b->stream, &cs) == hipSuccess && cs == hipStreamCaptureStatusNone;
+    return ws_ready(b, krk::gemm_mfma_group_workspace(rows, n_out, n, n_in, false));
 }
 
 int run_mfma_group(krk_backend *b, void *const out[], const void *x, const void *const w[], int wt,
@@ -509,7 +521,8 @@ int krk_gemm_group(krk_backend *b, void *const out[], const void *x, const void 
         bool one = uniform && n_mat <= krk::kMaxSegs;
         for (int m = 0; m < n_mat && one; m++)
             one = (!xs || xs[m] == xs[0]) && rows_path(b, t0, n_out[m], n_in, rows, w[m]);
-        one = one && krk::gemm_rows_tiles_ok(t0, n_in, n_out, n_mat, b->tile_cnt != nullptr);
+        one = one && krk::gemm_rows_tiles_ok(t0, n_in, n_out, n_mat, b->tile_cnt != nullptr) &&
+              ws_ready(b, rows_scratch(b, n_out, n_in, n_mat, rows));
         if (one) return run_rows(b, out, xs ? xs[0] : x, w, t0, n_out, n_in, n_mat, rows, nullptr, 0);
         if (group_mfma(b, w, t0, n_out, n_in, n_mat, rows, xs, uniform))
             return run_mfma_group(b, out, xs ? xs[0] : x, w, t0, n_out, n_in, n_mat, rows);

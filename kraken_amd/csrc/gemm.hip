@@ -22,8 +22,10 @@
 //     weight tiles in its own L2;
 //   * split-K (z dimension) when the tile count cannot fill 256 CUs: two
 //     splits summed inside the GEMM by the one that arrives second (per-tile
-//     counters), more splits as f32 partials summed in a fixed order by a
-//     second kernel.
+//     counters), more splits, of equal or unequal length, as f32 partials
+//     summed in a fixed order by a second kernel;
+//   * f32 rows of the five common formats are rounded to f16 once, before the
+//     GEMM.
 //
 // int8 path (KRK_PATH_INT8, Q8_0 weights only): activations quantized per 32
 // with the host rule (quantize_q8_32_d), v_mfma_i32_32x32x32_i8 per 32-value

@@ -11,8 +11,8 @@
 // ramp and tail (the preparation's launch, the first loads' latency, the
 // waves' sums).  Measured, Q4_K f16 rows: 4096 -> 14336 8 rows 19.4 -> 16.0 us,
 // 14336 -> 4096 8 rows 80.9 -> 20.8 us (6.7 us of HBM time each); the f16
-// expert layer (128 experts, 4096 / 1536, top 8) 160 tokens 9797 -> 435 us,
-// one token 233 -> 65 us.  What the layout buys:
+// expert layer (128 experts, 4096 / 1536, top 8) 160 tokens 9797 -> 420 us.
+// What the layout buys:
 //   * A workgroup owns 16 or 32 weight rows over all of K; its waves split K
 //     into contiguous slices of NBW 256-value blocks, and a wave requests
 //     every weight byte of its slice before any arithmetic, so no barrier or
@@ -22,9 +22,11 @@
 //     load 16 bytes a lane (the four lane rows cover whole 64-byte lines) and
 //     cross-row lane swaps hand each row its share; the activations are
 //     prepared in the order that leaves (rows_prep_kernel).
-//   * Nibble codes need no conversion: a nibble masked inside a 16-bit half
-//     is the f16 subnormal q 2^-24 (bits 0..3) or q 2^-20 (bits 4..7), which
-//     the matrix cores take exactly; five VALU operations serve eight codes.
+//   * Codes become f16 without conversions: a code placed in the mantissa of
+//     1024 or 64 is 1024 + q or 64 + q, and one packed f16 operation takes the
+//     constant off (with the sub-block's scale where scale x code is exact in
+//     f16).  Left as subnormals they cost precision: the matrix cores take
+//     them, but sums lose low bits (3.5e-6 against 2.7e-7).
 //   * Q4_K / Q5_K minimums: one more MFMA per block, the 6-bit mins against
 //     the activation rows' sub-block sums (three f16 planes, exact to 2^-33).
 #include <cstdint>

@@ -2,15 +2,20 @@
 // device pointer table (Backend::moe_dispatch, backend.hpp:1001-1009; the
 // reference's moe_table_* kernels, src/hip/kernels/moe_table.hpp:38-551).
 //
-// Q4_K banks with f32 activations run on the int8 matrix cores (digit-plane
-// activations): one token takes two launches of the register-streaming
-// GEMV (gate/up per slot, down over the concatenated slots); more tokens
-// take the plan, then expert-major runs of the same kernel -- one grid row
-// per active expert, whose banks are loaded once and applied to each of its
-// tokens in turn -- for gate/up and for down, then the ordered reduce (step 4
-// below).  Other f32 cases: one token takes two VALU launches; more tokens
-// take the plan path, none of its launches per expert and none waiting on
-// the host:
+// One token of Q4_K banks (Q4_K or Q6_K down) runs on the int8 matrix cores
+// (digit-plane activations), without a plan: f32 in two launches of the
+// register-streaming GEMV (gate/up per slot, down over the concatenated
+// slots), f16 (Q4_K down) in four (gate/up, the row scales, down per slot, the
+// slot-order reduce).  Several f32 tokens on a few experts each take the plan,
+// then expert-major runs of the same kernel -- one grid row per active expert,
+// whose banks are loaded once and applied to each of its tokens in turn --
+// for gate/up and for down, then the ordered reduce (step 4 below).  f32
+// batches of 32 tokens or more take the grouped expert GEMM (gemm.hip) where
+// f16 products are allowed.  Other layers of one gate/up type and one down
+// type, and f16 activations at any token count, take the plan, the rows
+// kernel (gemm_rows.hip; moe_rows below) and the reduce.  What is left runs on
+// the VALU: one f32 token in two launches; more tokens in the plan path, none
+// of its launches per expert and none waiting on the host:
 //   1. plan      one workgroup: expert-major plan of the (token, slot) pairs,
 //                the active-expert list in ascending id (with each expert's
 //                banks and plan range), and each pair's plan position;
@@ -23,8 +28,8 @@
 //                fma(w, part, acc) -- the order and the fused add of the host
 //                loop (engine.cpp:12360-12700, scatter_axpy_rows
 //                backend_cpu.cpp:3193-3217).
-// f16 activations (the reference GPU backend's act_type) take the plan path
-// at every token count with the reference GPU's rounding points
+// f16 activations (the reference GPU backend's act_type) have the reference
+// GPU's rounding points on every path
 // (moe_table.hpp:250-305, 418-441, 536-551): gate/up dots rounded to f16
 // before silu, a row-scale pass (power of two keeping the row within f16,
 // midf = f16(mid / scale)), down on midf, and a reduce that adds
